@@ -18,7 +18,7 @@
 // P2 + p and south node P2 - 1 - p; degrees split by parity, n = 2k + q.
 //   Tinv [q][KP][P2p]  Pt_n(mu_p)          (inverse; pairs fastest)
 //   Tfwd [q][P2p][KR]  (w_p/2) Pt_n(mu_p)  (forward; degrees fastest)
-// Both directions are GEMMs on v_mfma_f64_16x16x4f64, one wavefront per
+// Both directions are GEMMs on v_mfma_f64_16x16x4f64, one workgroup per
 // 16 x 16 output tile (the EBM's single field uses one column of it).
 #include <cstring>
 #include <new>
@@ -60,61 +60,110 @@ __global__ void zonal_table_kernel(int N, int P2, int P2p, int KP, int KR, const
   }
 }
 
-// l_y: wave = (parity q, 16-degree tile, 16-field tile); K runs over pairs.
-__global__ __launch_bounds__(64) void zonal_fwd_kernel(const double *__restrict__ y, double *__restrict__ l,
-                                                        const double *__restrict__ Tfwd, int N, int jm, int P2,
-                                                        int P2p, int KR, int nrt, int nf) {
+// Both directions: a workgroup of nw wavefronts owns one 16 x 16 output tile
+// (for l_y of one parity) and splits its K loop over the waves, wave w taking
+// the steps w, w + nw, ... (4 K values each) kZonalAhead at a time with all
+// their loads issued before the first MFMA; the partial tiles meet in LDS and
+// are added in wave order in FP64.  Bound by latency: one tile's K loop run by
+// a single wave is a chain of load-MFMA steps, and a one-field call of degree
+// 1024 has only 33-66 tiles.  Measured at nmax = jm = 1024, one field: l_y
+// 32.9 -> 5.5 us, y_l 61.2 -> 7.5 us (the tables are
+// 4.3 MB each; 20 steps ahead for y_l, one round of loads: 9.3 us).
+// nw depends on the plan alone, so a field's result does not depend on nf.
+constexpr int kZonalAhead = 8;
+constexpr int kZonalMaxWaves = 16;
+
+// Partial tiles to LDS, red[wave][item][lane]; returns after the barrier.
+__device__ __forceinline__ void zonal_put(double *red, int slot, int lane, const d4 &acc) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[(slot * 4 + i) * 64 + lane] = acc[i];
+}
+// element e = item * 64 + lane of the sum of the n partial tiles from slot0 on
+__device__ __forceinline__ double zonal_sum(const double *red, int slot0, int n, int e) {
+  double v = red[slot0 * 256 + e];
+  for (int w = 1; w < n; ++w) v += red[(slot0 + w) * 256 + e];
+  return v;
+}
+
+// l_y: workgroup = (parity q, 16-degree tile, 16-field tile); K runs over pairs.
+__global__ __launch_bounds__(64 * kZonalMaxWaves) void zonal_fwd_kernel(
+    const double *__restrict__ y, double *__restrict__ l, const double *__restrict__ Tfwd, int N, int jm,
+    int P2, int P2p, int KR, int nrt, int nf) {
+  extern __shared__ double red[];  // [nw][4][64]
   const int b = blockIdx.x, q = b & 1, rt = (b >> 1) % nrt, ct = (b >> 1) / nrt;
-  const int lane = threadIdx.x, r16 = lane & 15, kq = lane >> 4;
+  const int wave = wave_id(), nw = blockDim.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
   const int f = ct * 16 + r16;
   const double *__restrict__ T = Tfwd + (size_t)q * P2p * KR + rt * 16 + r16;
   const double *__restrict__ yf = y + (size_t)(f < nf ? f : 0) * jm;
   const double sgn = q ? -1.0 : 1.0;
+  const int nsteps = P2p >> 2;
   d4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int s = 0; s < (P2p >> 2); ++s) {
-    const int p = s * 4 + kq;
-    const double a = T[(size_t)p * KR];
-    double v = 0.0;
-    if (p < P2 && f < nf) v = yf[P2 + p] + sgn * yf[P2 - 1 - p];
-    acc = mfma16x4(a, v, acc);
-  }
-  if (f >= nf) return;
-  const int kn = q ? (N + 1) >> 1 : (N + 2) >> 1;  // degrees of this parity
+  for (int s0 = wave; s0 < nsteps; s0 += nw * kZonalAhead) {
+    // steps past the end and pairs past P2 load valid addresses and count as 0
+    double a[kZonalAhead], yn[kZonalAhead], ys[kZonalAhead];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = rt * 16 + i * 4 + kq;
-    if (k < kn) l[(size_t)f * (N + 1) + 2 * k + q] = acc[i];
+    for (int j = 0; j < kZonalAhead; ++j) {
+      const int s = s0 + j * nw, p = (s < nsteps ? s : 0) * 4 + kq, pc = p < P2 ? p : 0;
+      a[j] = T[(size_t)p * KR];
+      yn[j] = yf[P2 + pc];
+      ys[j] = yf[P2 - 1 - pc];
+    }
+#pragma unroll
+    for (int j = 0; j < kZonalAhead; ++j) {
+      const int s = s0 + j * nw;
+      const double v = s < nsteps && s * 4 + kq < P2 && f < nf ? yn[j] + sgn * ys[j] : 0.0;
+      if (s < nsteps) acc = mfma16x4(a[j], v, acc);
+    }
+  }
+  zonal_put(red, wave, lane, acc);
+  __syncthreads();
+  const int kn = q ? (N + 1) >> 1 : (N + 2) >> 1;  // degrees of this parity
+  for (int e = threadIdx.x; e < 256; e += blockDim.x) {
+    // item i of lane ln: degree row 4 i + ln / 16, field ln % 16
+    const int k = rt * 16 + (e >> 6) * 4 + ((e & 63) >> 4), fo = ct * 16 + (e & 15);
+    if (k < kn && fo < nf) l[(size_t)fo * (N + 1) + 2 * k + q] = zonal_sum(red, 0, nw, e);
   }
 }
 
-// y_l: wave = (16-pair tile, 16-field tile); even and odd degrees in two
-// accumulators, then north = even + odd, south = even - odd.
-__global__ __launch_bounds__(64) void zonal_inv_kernel(const double *__restrict__ l, double *__restrict__ y,
-                                                        const double *__restrict__ Tinv, int N, int jm, int P2,
-                                                        int P2p, int KP, int nrt, int nf) {
+// y_l: workgroup = (16-pair tile, 16-field tile); the first half of the waves
+// sums the even degrees, the second half the odd ones, then north = even +
+// odd, south = even - odd.
+__global__ __launch_bounds__(64 * kZonalMaxWaves) void zonal_inv_kernel(
+    const double *__restrict__ l, double *__restrict__ y, const double *__restrict__ Tinv, int N, int jm,
+    int P2, int P2p, int KP, int nrt, int nf) {
+  extern __shared__ double red[];  // [nw][4][64], even halves first
   const int b = blockIdx.x, rt = b % nrt, ct = b / nrt;
-  const int lane = threadIdx.x, r16 = lane & 15, kq = lane >> 4;
+  const int wave = wave_id(), nh = blockDim.x >> 7, lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  const int q = wave >= nh ? 1 : 0, w = wave - q * nh;
   const int f = ct * 16 + r16;
   const double *__restrict__ lf = l + (size_t)(f < nf ? f : 0) * (N + 1);
-  d4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+  const double *__restrict__ T = Tinv + (size_t)q * KP * P2p + rt * 16 + r16;
+  const int nsteps = KP >> 2;
+  d4 acc = {0.0, 0.0, 0.0, 0.0};
+  for (int s0 = w; s0 < nsteps; s0 += nh * kZonalAhead) {
+    double a[kZonalAhead], v[kZonalAhead];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const double *__restrict__ T = Tinv + (size_t)q * KP * P2p + rt * 16 + r16;
-    for (int s = 0; s < (KP >> 2); ++s) {
-      const int k = s * 4 + kq, n = 2 * k + q;
-      const double a = T[(size_t)k * P2p];
-      const double v = (n <= N && f < nf) ? lf[n] : 0.0;
-      acc[q] = mfma16x4(a, v, acc[q]);
+    for (int j = 0; j < kZonalAhead; ++j) {
+      const int s = s0 + j * nh, k = (s < nsteps ? s : 0) * 4 + kq, n = 2 * k + q;
+      a[j] = T[(size_t)k * P2p];
+      v[j] = lf[n <= N ? n : 0];
+    }
+#pragma unroll
+    for (int j = 0; j < kZonalAhead; ++j) {
+      const int s = s0 + j * nh;
+      const double x = s < nsteps && 2 * (s * 4 + kq) + q <= N && f < nf ? v[j] : 0.0;
+      if (s < nsteps) acc = mfma16x4(a[j], x, acc);
     }
   }
-  if (f >= nf) return;
-  double *__restrict__ yf = y + (size_t)f * jm;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int p = rt * 16 + i * 4 + kq;
-    if (p < P2) {
-      yf[P2 + p] = acc[0][i] + acc[1][i];
-      yf[P2 - 1 - p] = acc[0][i] - acc[1][i];
+  zonal_put(red, wave, lane, acc);
+  __syncthreads();
+  for (int e = threadIdx.x; e < 256; e += blockDim.x) {
+    const int p = rt * 16 + (e >> 6) * 4 + ((e & 63) >> 4), fo = ct * 16 + (e & 15);
+    if (p < P2 && fo < nf) {
+      const double ev = zonal_sum(red, 0, nh, e), od = zonal_sum(red, nh, nh, e);
+      double *__restrict__ yf = y + (size_t)fo * jm;
+      yf[P2 + p] = ev + od;
+      yf[P2 - 1 - p] = ev - od;
     }
   }
 }
@@ -174,16 +223,26 @@ int zonal_check(const sht_zonal *z, const void *a, const void *b, int nf, const 
   return SHT_OK;
 }
 
+// Waves that share a tile of nsteps K steps: about kZonalAhead steps each, so
+// that a wave's loads are one round, and an even number (y_l deals halves to
+// the two parities).
+int zonal_waves(int nsteps) {
+  const int nw = roundup((nsteps + kZonalAhead - 1) / kZonalAhead, 2);
+  return nw < kZonalMaxWaves ? nw : kZonalMaxWaves;
+}
+
 int zonal_fwd(const sht_zonal *z, const double *y, double *l, int nf, hipStream_t s) {
-  const int nrt = z->KR / 16, nct = (nf + 15) / 16;
-  zonal_fwd_kernel<<<2 * nrt * nct, 64, 0, s>>>(y, l, z->Tfwd, z->N, z->jm, z->P2, z->P2p, z->KR, nrt, nf);
+  const int nrt = z->KR / 16, nct = (nf + 15) / 16, nw = zonal_waves(z->P2p / 4);
+  zonal_fwd_kernel<<<2 * nrt * nct, 64 * nw, sizeof(double) * 256 * nw, s>>>(
+      y, l, z->Tfwd, z->N, z->jm, z->P2, z->P2p, z->KR, nrt, nf);
   SHT_HIP(hipGetLastError());
   return SHT_OK;
 }
 
 int zonal_inv(const sht_zonal *z, const double *l, double *y, int nf, hipStream_t s) {
-  const int nrt = z->P2p / 16, nct = (nf + 15) / 16;
-  zonal_inv_kernel<<<nrt * nct, 64, 0, s>>>(l, y, z->Tinv, z->N, z->jm, z->P2, z->P2p, z->KP, nrt, nf);
+  const int nrt = z->P2p / 16, nct = (nf + 15) / 16, nw = zonal_waves(2 * (z->KP / 4));
+  zonal_inv_kernel<<<nrt * nct, 64 * nw, sizeof(double) * 256 * nw, s>>>(
+      l, y, z->Tinv, z->N, z->jm, z->P2, z->P2p, z->KP, nrt, nf);
   SHT_HIP(hipGetLastError());
   return SHT_OK;
 }

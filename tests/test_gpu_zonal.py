@@ -92,3 +92,21 @@ def test_zonal_vs_oracle(nm, jm, nf):
     if nm < jm:
         assert np.abs(z.l_y(z.y_l(l)) - l).max() < 1e-12
     z.close()
+
+
+@pytest.mark.parametrize("nm,jm,nf", [(31, 32, 1), (129, 260, 17), (255, 258, 16), (2047, 2048, 2)])
+def test_zonal_waves_per_tile(nm, jm, nf):
+    """K loops of one step a wave, of a part-filled round, and of more than one
+    round: the oracle's values, and a field's result is the same alone."""
+    rng = np.random.default_rng(jm)
+    mu, w, cl = oracle.gauss(jm)
+    Pt = oracle.legendre_column(nm, 0, mu, cl)
+    y = rng.standard_normal((nf, jm))
+    l = rng.standard_normal((nf, nm + 1)) / np.sqrt(1.0 + np.arange(nm + 1))
+    z = shtamd.Zonal(nm, jm, kmax=nf)
+    lo, yo = z.l_y(y), z.y_l(l)
+    l_ref, y_ref = 0.5 * (y * w) @ Pt.T, l @ Pt
+    assert np.linalg.norm(lo - l_ref) / np.linalg.norm(l_ref) < 1e-12
+    assert np.linalg.norm(yo - y_ref) / np.linalg.norm(y_ref) < 1e-12
+    assert np.array_equal(z.l_y(y[-1]), lo[-1]) and np.array_equal(z.y_l(l[-1]), yo[-1])
+    z.close()
