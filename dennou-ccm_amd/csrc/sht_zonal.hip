@@ -67,13 +67,13 @@ __global__ void zonal_table_kernel(int N, int P2, int P2p, int KP, int KR, const
 // are added in wave order in FP64.  Bound by latency: one tile's K loop run by
 // a single wave is a chain of load-MFMA steps, and a one-field call of degree
 // 1024 has only 33-66 tiles.  Measured at nmax = jm = 1024, one field: l_y
-// 32.9 -> 5.5 us, y_l 61.2 -> 7.5 us (the tables are
-// 4.3 MB each; 20 steps ahead for y_l, one round of loads: 9.3 us).
+// 32.9 -> 5.5 us, y_l 61.2 -> 7.5 us (the tables are 4.3 MB each; 20 steps
+// ahead for y_l, one round of loads: 9.3 us).
 // nw depends on the plan alone, so a field's result does not depend on nf.
 constexpr int kZonalAhead = 8;
 constexpr int kZonalMaxWaves = 16;
 
-// Partial tiles to LDS, red[wave][item][lane]; returns after the barrier.
+// A partial tile to LDS, red[slot][item][lane].
 __device__ __forceinline__ void zonal_put(double *red, int slot, int lane, const d4 &acc) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) red[(slot * 4 + i) * 64 + lane] = acc[i];
