@@ -5,7 +5,7 @@
 // for d = 1..ndata, fields contiguous per point (Fortran send_data(:, d)).
 //
 // The triplets are regrouped at creation by receiving point (CSR), keeping
-// the original order within each row, and one thread sums one (row, field)
+// the original order within each row, and one thread sums each (row, field)
 // with separately rounded multiply and add in that order: the same operations
 // in the same order as the reference loop, so results are bitwise equal to an
 // unfused evaluation of it (no atomics, no fused multiply-add).
@@ -25,6 +25,15 @@ struct sht_remap {
 namespace sht {
 namespace {
 
+// One thread sums one row for ND fields (the last group of a call has fewer):
+// row offsets, columns and coefficients are loaded once for the group, and
+// kRemapAhead entries' columns, then their ND gathers each, are in flight at a
+// time, where one load at a time is a chain row -> column -> value per entry.
+// 32,768 rows of 4 entries, back to back: 12 fields 5.2 -> 3.9 us, 40 fields
+// 13.4 -> 7.5 us; 131,072 rows, 40 fields 45.4 -> 22.6 us.  Small calls run
+// single fields (ND = 1): 8,192 rows, 12 fields 3.1 -> 2.9 us.
+constexpr int kRemapAhead = 4;
+template <int ND>
 __global__ __launch_bounds__(256) void remap_kernel(const int *__restrict__ row,
                                                     const int *__restrict__ col,
                                                     const double *__restrict__ val,
@@ -35,16 +44,45 @@ __global__ __launch_bounds__(256) void remap_kernel(const int *__restrict__ row,
   // into one fused multiply-add (the operations must be written here, in the
   // pragma's scope: __dmul_rn/__dadd_rn are contracted at their definition)
 #pragma clang fp contract(off)
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)nrecv * ndata) return;
-  const int r = (int)(t % nrecv), d = (int)(t / nrecv);
-  const double *__restrict__ s = send + (size_t)d * nsend;
-  double acc = 0.0;
-  for (int i = row[r]; i < row[r + 1]; ++i) {
-    const double prod = s[col[i]] * val[i];
-    acc = acc + prod;
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t total = (int64_t)nrecv * ((ndata + ND - 1) / ND);
+  if (t >= total) return;
+  // 32-bit division where it suffices
+  const int g = total <= UINT32_MAX ? (int)((uint32_t)t / (uint32_t)nrecv) : (int)(t / nrecv);
+  const int r = (int)(t - (int64_t)g * nrecv), d0 = g * ND;
+  const int nd = ndata - d0 < ND ? ndata - d0 : ND;
+  const double *__restrict__ s = send + (size_t)d0 * nsend;
+  double acc[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) acc[d] = 0.0;
+  const int end = row[r + 1];
+  for (int i0 = row[r]; i0 < end; i0 += kRemapAhead) {
+    // entries past the row's end repeat its last one and are not added
+    int c[kRemapAhead];
+    double w[kRemapAhead], x[kRemapAhead][ND];
+#pragma unroll
+    for (int u = 0; u < kRemapAhead; ++u) {
+      const int i = i0 + u < end ? i0 + u : end - 1;
+      c[u] = col[i];
+      w[u] = val[i];
+    }
+#pragma unroll
+    for (int u = 0; u < kRemapAhead; ++u)
+#pragma unroll
+      for (int d = 0; d < ND; ++d) x[u][d] = s[(size_t)(d < nd ? d : 0) * nsend + c[u]];
+#pragma unroll
+    for (int u = 0; u < kRemapAhead; ++u) {
+      if (i0 + u >= end) break;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        const double prod = x[u][d] * w[u];
+        acc[d] = acc[d] + prod;
+      }
+    }
   }
-  recv[(size_t)d * nrecv + r] = acc;
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+    if (d < nd) recv[(size_t)(d0 + d) * nrecv + r] = acc[d];
 }
 
 void remap_release(sht_remap *m) {
@@ -114,7 +152,10 @@ int sht_remap_apply_dev(const sht_remap *m, const double *send, double *recv, in
   if (!send || !recv || ndata < 1) return fail(SHT_ERR_INVALID, "sht_remap_apply_dev: bad arguments");
   const int64_t n = (int64_t)m->nrecv * ndata;
   if (n > (int64_t)INT32_MAX * 128) return fail(SHT_ERR_INVALID, "sht_remap_apply_dev: too many outputs");
-  remap_kernel<<<(unsigned)((n + 255) / 256), 256, 0, (hipStream_t)stream>>>(
+  // groups of 4 fields where that still gives each CU a workgroup
+  const bool wide = (int64_t)m->nrecv * (ndata / 4) >= 256 * 256;
+  const int64_t nt = wide ? (int64_t)m->nrecv * ((ndata + 3) / 4) : n;
+  (wide ? remap_kernel<4> : remap_kernel<1>)<<<(unsigned)((nt + 255) / 256), 256, 0, (hipStream_t)stream>>>(
       m->row, m->col, m->val, send, recv, m->nsend, m->nrecv, ndata);
   SHT_HIP(hipGetLastError());
   return SHT_OK;

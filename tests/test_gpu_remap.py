@@ -76,3 +76,20 @@ def test_remap_argument_checks():
     torch.cuda.synchronize()
     assert torch.count_nonzero(out) == 0
     r.close()
+
+
+@pytest.mark.parametrize("nrecv,ndata", [(3, 2), (40000, 11), (40000, 13), (40000, 16)])
+def test_remap_field_groups_bitwise(nrecv, ndata):
+    """Rows of 0 to 9 entries, groups of one and of four fields (part-filled ones too)."""
+    rng = np.random.default_rng(nrecv + ndata)
+    nsend = 1000
+    ri = np.repeat(np.arange(nrecv), np.arange(nrecv) % 10)
+    si = rng.integers(0, nsend, ri.size)
+    cf = rng.standard_normal(ri.size)
+    send = rng.standard_normal((ndata, nsend))
+    r = shtamd.Remap(si, ri, cf, nsend, nrecv)
+    out = torch.full((ndata, nrecv), np.nan, dtype=torch.float64, device="cuda")
+    r.apply(torch.from_numpy(send).cuda(), out, ndata)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), oracle.remap(si, ri, cf, nrecv, send))
+    r.close()
