@@ -156,11 +156,12 @@ inline int avr_threads(int n) {
   return t < 1024 ? t : 1024;
 }
 
-// out = (-n(n+1))^power in on the canonical rows.  Every block makes the
-// factors of all degrees once (LDS); a thread then has AHEAD complex values in
-// flight while it finds their degrees (lapla_degree).  T85, 97
-// fields (5.8 MB each way), back to back: 13.5 -> 4.9 us with a search for m
-// and a power per value before.
+// out = (-n(n+1))^power in on the canonical rows, one complex value per thread.
+// Every block makes the factors of all degrees once (LDS) while its loads are
+// in flight, and finds a value's degree in closed form (lapla_degree).  T85, 97
+// fields (5.8 MB each way), back to back: 13.8 -> 3.9 us with a search for m
+// and a power per value before (four values per thread: 5.3 us, and slower at
+// every size up to 11 M values).
 // degree of canonical row k: off(m) = m (2N + 3 - m) / 2, so the largest m with
 // off(m) <= k is the floor of the smaller root of m^2 - (2N + 3) m + 2k; the
 // FP32 root is within one of it (all terms are below 2^24) and is corrected
@@ -173,14 +174,11 @@ __device__ __forceinline__ int lapla_degree(int N, int k) {
   while (m < N && off(m + 1) <= k) ++m;
   return m + k - off(m);
 }
-template <int AHEAD>
 __global__ __launch_bounds__(256) void lapla_kernel(const double2 *in, double2 *out, int N, int nf,
                                                     int power, int64_t total) {
   __shared__ double fac[256];  // N <= 255
-  const int64_t t0 = (int64_t)blockIdx.x * (256 * AHEAD) + threadIdx.x;
-  double2 v[AHEAD];
-#pragma unroll
-  for (int q = 0; q < AHEAD; ++q) v[q] = t0 + q * 256 < total ? in[t0 + q * 256] : make_double2(0.0, 0.0);
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const double2 v = t < total ? in[t] : make_double2(0.0, 0.0);
   if ((int)threadIdx.x <= N) {
     const int n = threadIdx.x;
     const double e = -(double)n * (n + 1);
@@ -194,28 +192,19 @@ __global__ __launch_bounds__(256) void lapla_kernel(const double2 *in, double2 *
     fac[n] = x;
   }
   __syncthreads();
-#pragma unroll
-  for (int q = 0; q < AHEAD; ++q) {
-    const int64_t t = t0 + q * 256;
-    if (t < total) {
-      // 32-bit division where it suffices
-      const int k = total <= UINT32_MAX ? (int)((uint32_t)t / (uint32_t)nf) : (int)(t / nf);
-      const double x = fac[lapla_degree(N, k)];
-      out[t] = make_double2(x * v[q].x, x * v[q].y);
-    }
-  }
+  if (t >= total) return;
+  // 32-bit division where it suffices
+  const int k = total <= UINT32_MAX ? (int)((uint32_t)t / (uint32_t)nf) : (int)(t / nf);
+  const double x = fac[lapla_degree(N, k)];
+  out[t] = make_double2(x * v.x, x * v.y);
 }
-
-// values from which a thread takes four
-constexpr int64_t kLaplaWide = 0;
 
 }  // namespace
 
 int launch_spec_lapla(const Plan &p, const double *in, double *out, int power, int nf,
                       hipStream_t s) {
   const int64_t n = (int64_t)p.K * nf;
-  const int ahead = n < kLaplaWide ? 1 : 4;
-  (ahead == 1 ? lapla_kernel<1> : lapla_kernel<4>)<<<(unsigned)((n + 256 * ahead - 1) / (256 * ahead)), 256, 0, s>>>(
+  lapla_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
       reinterpret_cast<const double2 *>(in), reinterpret_cast<double2 *>(out), p.N, nf, power, n);
   SHT_HIP(hipGetLastError());
   return SHT_OK;
