@@ -117,7 +117,7 @@ __global__ __launch_bounds__(kThreadsOf<C>) void fft_fwd_kernel(FwdIO<TF> io,
       A = make_double2(-m * A.y, m * A.x);
     }
     if (m == 0) S.y = A.y = 0.0;
-    TF *o = four + ft.off(m, M1, nf) + 2 * g;
+    TF *o = four + ft.off(m, M1, P2) + 2 * g;
     store_pair(o, S);
     store_pair(o + 2 * FourTile<G>::GL, A);
   }

@@ -113,11 +113,10 @@ struct FourTile {
     p = rest % P2;
     fgr = (rest / P2) * KS + sub;
   }
-  // offset of (m, parity 0, the block's first field) for nf fields; parity
-  // 1 follows 2 GL values later
-  __device__ __forceinline__ size_t off(int m, int M1, int nf) const {
-    const int nfg = (nf + GL - 1) / GL;
-    return ((((size_t)p * nfg + fgr / KS) * M1 + m) * 2) * (2 * GL) + (fgr % KS) * (2 * G);
+  // offset of (m, parity 0, the block's first field); parity 1 follows 2 GL
+  // values later
+  __device__ __forceinline__ size_t off(int m, int M1, int P2) const {
+    return ((((size_t)(fgr / KS) * P2 + p) * M1 + m) * 2) * (2 * GL) + (fgr % KS) * (2 * G);
   }
 };
 // FFT tiles of a call with nf fields
@@ -295,7 +294,7 @@ __device__ __forceinline__ void fft_inv_tile(double2 *buf, double2 *twl, const d
     const int idx = tid + q * kThreads;
     const int m = idx / G, g = idx % G, f = f0 + g;
     const bool ok = m < M1 && f < nf;
-    const TF *e = src + ft.off(ok ? m : 0, M1, nf) + (ok ? 2 * g : 0);
+    const TF *e = src + ft.off(ok ? m : 0, M1, P2) + (ok ? 2 * g : 0);
     Er[q] = load_four_raw<COH>(e);
     Or[q] = load_four_raw<COH>(e + 2 * FourTile<G>::GL);
   }
