@@ -204,20 +204,15 @@ static int spec_to_grad(Plan &p, const double *spec, double *grid, double *glon,
 // Flux divergence (1/cos) dA/dlon + (1/cos) d(B cos)/dlat to spectra, FP64 in
 // every precision form: A's Fourier coefficients times i m / cos meet the
 // value table, B's times 1 / cos meet -(w/2)(1-mu^2) dPt/dmu (the lat term
-// integrated by parts) with the parity slots swapped; the second GEMM adds
-// into the first's output.
+// integrated by parts) with the parity slots swapped, both sums in one
+// Legendre launch.
 static int grid_to_div(Plan &p, const double *a, const double *b, double *spec, int nf,
                        hipStream_t s) {
   double *fa = a ? p.four : nullptr;
   double *fb = b ? (a ? p.four2 : p.four) : nullptr;
   int rc = timed(p, SHT_STAGE_FFT_FWD, s, [&] { return launch_fft_fwd_div(p, a, fa, b, fb, nf, s); });
   if (rc) return rc;
-  return timed(p, SHT_STAGE_LEG_FWD, s, [&] {
-    int r = SHT_OK;
-    if (a) r = launch_leg_fwd_f64_table(p, p.Pfwd, fa, spec, false, false, nf, s);
-    if (!r && b) r = launch_leg_fwd_f64_table(p, p.Hfwd, fb, spec, true, a != nullptr, nf, s);
-    return r;
-  });
+  return timed(p, SHT_STAGE_LEG_FWD, s, [&] { return launch_leg_fwd_f64_div(p, fa, fb, spec, nf, s); });
 }
 
 // One direction of the transform on a plan (used by the ensemble batches).

@@ -40,7 +40,8 @@ int fail(int code, const std::string &msg);
 //   Hfwd  per m: [par 2][P2p][KR(m)]  -(w_p/2) (1-mu^2) dPt/dmu (forward DivLat)
 //   Pfwd  per m: [par 2][P2p][KR(m)]  (w_p/2) Pt_n^m(mu_p)  (forward, k fastest)
 //   KP(m) = roundup(ceil((N-m+1)/2), 4), KR(m) = roundup(ceil((N-m+1)/2), 16),
-//   padding entries are zero.
+//   padding entries are zero.  Pinv and Hinv are kStepSlack steps (of 4 rows)
+//   longer than their last m: kernels load whole chunks of kStepSlack + 1 steps.
 //
 //   four  [nfg][P2][N+1][par 2][2G]  the Fourier intermediate: per field group
 //         (G = max(2048/im, 8) fields, nfg = ceil(nf/G) groups), latitude pair
@@ -56,6 +57,8 @@ int fail(int code, const std::string &msg);
 // Mixed-precision plans also hold the tables split into 16-bit pieces in the
 // matrix-core operand layout (sht_legendre_mixed.hip) and use an FP32 Fourier
 // intermediate.
+
+constexpr int kStepSlack = 3;
 
 struct Plan {
   int N = 0, im = 0, jm = 0, P2 = 0, P2p = 0, K = 0, kmax = 0, prec = 0, flags = 0;
@@ -281,10 +284,9 @@ int launch_leg_fwd_f64_shape(const Plan &p, int shape, const double *four, doubl
 int launch_leg_inv_f64(const Plan &p, const double *spec, double *four, double *four2,
                        bool value_table, bool deriv_table, int nf, hipStream_t s);
 int launch_leg_fwd_f64(const Plan &p, const double *four, double *spec, int nf, hipStream_t s);
-// Forward Legendre (K-split shape) with any forward-layout table; swap = take the
-// opposite parity slot of the Fourier data (H tables), accumulate = add into spec.
-int launch_leg_fwd_f64_table(const Plan &p, const double *table, const double *four, double *spec,
-                             bool swap, bool accumulate, int nf, hipStream_t s);
+// Divergence analysis: spec = Pfwd fa + Hfwd fb with fb's parity slots swapped (either may be NULL)
+int launch_leg_fwd_f64_div(const Plan &p, const double *fa, const double *fb, double *spec, int nf,
+                           hipStream_t s);
 // spec_out = (-n(n+1))^power spec_in (negative powers leave n = 0 at zero)
 int launch_spec_lapla(const Plan &p, const double *in, double *out, int power, int nf, hipStream_t s);
 

@@ -171,6 +171,7 @@ int build_tables(Plan &p) {
   SHT_PLAN_ALLOC(p, &p.twid, sizeof(double) * 2 * p.im);
   SHT_PLAN_ALLOC(p, &p.zero, sizeof(double) * 64);
   SHT_HIP(hipMemset(p.zero, 0, sizeof(double) * 64));
+  ti += (size_t)kStepSlack * 4 * p.P2p;  // see kStepSlack
   SHT_PLAN_ALLOC(p, &p.Pinv, sizeof(double) * ti);
   SHT_PLAN_ALLOC(p, &p.Pfwd, sizeof(double) * tf);
   if (p.flags & SHT_FLAG_GRAD) SHT_PLAN_ALLOC(p, &p.Hinv, sizeof(double) * ti);

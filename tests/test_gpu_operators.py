@@ -140,3 +140,16 @@ def test_operator_argument_checks():
     torch.cuda.synchronize()
     assert torch.count_nonzero(s) == 0
     p.close()
+
+
+@pytest.mark.parametrize("N,im,jm,nf", [(0, 16, 2, 3), (31, 64, 48, 17), (127, 256, 192, 8), (201, 512, 202, 3), (255, 512, 512, 9)])
+def test_divergence_waves_and_units(N, im, jm, nf):
+    """One to two units per wave of four and of eight waves, the smallest and largest LDS blocks."""
+    rng = np.random.default_rng(N)
+    a, b = rng.standard_normal((2, nf, jm, im))
+    ref = oracle.Plan(N, im, jm)
+    p = shtamd.Plan(N, im, jm, nf, flags=shtamd.FLAG_GRAD)
+    for aa, bb in ((a, b), (a, None), (None, b)):
+        got, want = gpu_div(p, aa, bb, nf), ref.grid_to_div(aa, bb)
+        assert np.linalg.norm(got - want) <= TOL * max(np.linalg.norm(want), 1e-300) or not want.any()
+    p.close()
