@@ -208,10 +208,29 @@ def _dev(t, need: int, what: str) -> int | None:
     return _ptr(t)
 
 
+_raw_stream = None  # () -> handle of PyTorch's current stream
+
+
+def _current_stream() -> int:
+    """Handle of PyTorch's current stream on its current device.  Read through
+    PyTorch's own integer accessors where it has them: a torch.cuda.Stream
+    object per call costs 2.7 us, as much as a kernel launch, these 0.15 us."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+
+        torch.cuda.current_stream()  # initialises the device
+        handle, device = (getattr(torch._C, n, None) for n in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+        if handle and device:
+            _raw_stream = lambda: handle(device())  # noqa: E731
+        else:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream  # noqa: E731
+    return _raw_stream()
+
+
 def _stream_handle(stream) -> int | None:
     if stream is None:
-        import torch
-        return torch.cuda.current_stream().cuda_stream
+        return _current_stream()
     return getattr(stream, "cuda_stream", stream)
 
 
