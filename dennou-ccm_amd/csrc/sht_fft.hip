@@ -51,23 +51,17 @@ struct FwdIO {
 // workgroups of the last, partly empty field group evenly over the XCDs (T85,
 // 97 fields: inverse 9.8 -> 9.5 us); otherwise each XCD takes a contiguous
 // range of tiles, which measured ~1 % faster when blocks queue.
+// One tile of the stage (its block of C values, LDS at buf and twl).
 template <int L, typename TF, bool DIRECT, int C>
-__global__ __launch_bounds__(kThreadsOf<C>) void fft_fwd_kernel(FwdIO<TF> io,
-                                                                const double2 *__restrict__ tw,
-                                                                const double *__restrict__ coslat,
-                                                                int P2, int M1, int nf, int jm, int spread) {
-  const double *__restrict__ grid = io.src[blockIdx.y];
-  TF *__restrict__ four = io.dst[blockIdx.y];
-  const int mode = io.mode[blockIdx.y];
+__device__ __forceinline__ void fft_fwd_tile(double2 *buf, double2 *twl, const double *__restrict__ grid,
+                                             TF *__restrict__ four, int mode, const double2 *__restrict__ tw,
+                                             const double *__restrict__ coslat, int P2, int M1, int nf, int jm,
+                                             int tile, int tid) {
   constexpr int G = C / L;
   constexpr int kThreads = kThreadsOf<C>;
-  __shared__ double2 buf[kPaddedOf<C>];
-  __shared__ double2 twl[L];
-  const int tile = spread ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
   const FourTile<G> ft(tile, P2);
   const int p = ft.p, f0 = ft.fgr * G;
   const int jn = P2 + p, js = P2 - 1 - p;
-  const int tid = threadIdx.x;
   // the twiddles are loaded after the first ring loads are issued (one wait
   // covers both; loaded first, their wait held back every ring load)
   auto twiddles = [&] {
@@ -87,7 +81,7 @@ __global__ __launch_bounds__(kThreadsOf<C>) void fft_fwd_kernel(FwdIO<TF> io,
     if (i < M1 || i > L - M1) buf[px<L>(g * L + i)] = v;
   };
   if constexpr (DIRECT) {
-    fft_lds<L, -1, C>(buf, twl, ring, keep, threadIdx.x, twiddles);
+    fft_lds<L, -1, C>(buf, twl, ring, keep, tid, twiddles);
   } else {
     constexpr int NQ = C / kThreads;  // samples per thread
     double2 z[NQ];
@@ -100,7 +94,7 @@ __global__ __launch_bounds__(kThreadsOf<C>) void fft_fwd_kernel(FwdIO<TF> io,
 #pragma unroll
     for (int q = 0; q < NQ; ++q) buf[px<L>(tid + q * kThreads)] = z[q];
     __syncthreads();
-    fft_lds<L, -1, C>(buf, twl, [&](int g, int i) { return buf[px<L>(g * L + i)]; }, keep, threadIdx.x);
+    fft_lds<L, -1, C>(buf, twl, [&](int g, int i) { return buf[px<L>(g * L + i)]; }, keep, tid);
   }
   const double sc = 0.5 / L * (mode == 0 ? 1.0 : 1.0 / coslat[jn]);
   for (int idx = tid; idx < M1 * G; idx += kThreads) {
@@ -121,6 +115,19 @@ __global__ __launch_bounds__(kThreadsOf<C>) void fft_fwd_kernel(FwdIO<TF> io,
     store_pair(o, S);
     store_pair(o + 2 * FourTile<G>::GL, A);
   }
+}
+
+template <int L, typename TF, bool DIRECT, int C>
+__global__ __launch_bounds__(kThreadsOf<C>) void fft_fwd_kernel(FwdIO<TF> io,
+                                                                const double2 *__restrict__ tw,
+                                                                const double *__restrict__ coslat,
+                                                                int P2, int M1, int nf, int jm, int spread) {
+  __shared__ double2 buf[kPaddedOf<C>];
+  __shared__ double2 twl[L];
+  const int tile = spread ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
+  const int sel = blockIdx.y;
+  fft_fwd_tile<L, TF, DIRECT, C>(buf, twl, io.src[sel], io.dst[sel], io.mode[sel], tw, coslat, P2, M1, nf, jm, tile,
+                                 threadIdx.x);
 }
 
 
@@ -231,7 +238,81 @@ int inv_typed(const Plan &p, const TF *four, const TF *four2, double *grid, doub
   return fail(SHT_ERR_UNSUPPORTED, "im must be a power of two in [16, 2048]");
 }
 
+// ---- Several groups in one launch (sht_internal.h, MultiGroup): big blocks
+// only, at most kMultiMaxIm longitudes.  Each group's range of workgroups is
+// padded to a multiple of 8, so that its tiles meet the XCDs as in a launch of
+// their own.
+constexpr int kMultiMaxIm = 256;
+struct FftMulti {
+  int ng, spread;
+  struct Group {
+    const void *four;
+    double *grid;
+    const double2 *tw;
+    const double *coslat;
+    int blk0, nblk, im, P2, M1, nf, jm;
+  } g[kMaxMulti];
+};
+
+template <int L, typename TF, bool FWD, bool DIRECT>
+__device__ __forceinline__ void fft_multi_tile(double2 *buf, double2 *twl, const FftMulti::Group &g, int tile) {
+  TF *four = static_cast<TF *>(const_cast<void *>(g.four));
+  if constexpr (FWD)
+    fft_fwd_tile<L, TF, DIRECT, kFftBig>(buf, twl, g.grid, four, 0, g.tw, g.coslat, g.P2, g.M1, g.nf, g.jm, tile,
+                                         threadIdx.x);
+  else
+    fft_inv_tile<L, TF, false, kFftBig>(buf, twl, g.tw, four, g.grid, 0, g.coslat, g.P2, g.M1, g.nf, g.jm, tile,
+                                        threadIdx.x);
+}
+
+template <typename TF, bool FWD, bool DIRECT>
+__global__ __launch_bounds__(kThreads) void fft_multi_kernel(FftMulti a) {
+  __shared__ double2 buf[kLdsPadded];
+  __shared__ double2 twl[kMultiMaxIm];
+  const FftMulti::Group &g = a.g[multi_group(a, blockIdx.x)];
+  const int b = blockIdx.x - g.blk0;
+  if (b >= g.nblk) return;
+  const int tile = a.spread ? b : xcd_tile(b, g.nblk);
+  switch (g.im) {
+    case 16: return fft_multi_tile<16, TF, FWD, DIRECT>(buf, twl, g, tile);
+    case 32: return fft_multi_tile<32, TF, FWD, DIRECT>(buf, twl, g, tile);
+    case 64: return fft_multi_tile<64, TF, FWD, DIRECT>(buf, twl, g, tile);
+    case 128: return fft_multi_tile<128, TF, FWD, DIRECT>(buf, twl, g, tile);
+    case 256: return fft_multi_tile<256, TF, FWD, DIRECT>(buf, twl, g, tile);
+  }
+}
+
+template <bool FWD>
+int multi_launch(const MultiGroup *g, int n, hipStream_t s) {
+  FftMulti a{};
+  a.ng = n;
+  int nblk = 0, total = 0, resident = INT32_MAX;
+  for (int i = 0; i < n; ++i) {
+    const Plan &p = *g[i].p;
+    const FourGeom geo = multi_geom(p, g[i].nf);
+    const int gf = fft_group(p.im), nb = p.P2 * geo.nfg * (layout_group(gf) / gf);
+    a.g[i] = {p.four, g[i].grid, reinterpret_cast<const double2 *>(p.twid), p.coslat, nblk, nb, p.im, p.P2,
+              p.N + 1, g[i].nf, p.jm};
+    nblk += roundup(nb, 8);
+    total += nb;
+    resident = p.fft_fwd_resident[0] < resident ? p.fft_fwd_resident[0] : resident;
+  }
+  a.spread = total <= resident;
+  const bool f32 = g[0].p->prec != SHT_PREC_FP64;
+  void (*kern)(FftMulti);
+  if (FWD && a.spread)
+    kern = f32 ? fft_multi_kernel<float, FWD, true> : fft_multi_kernel<double, FWD, true>;
+  else
+    kern = f32 ? fft_multi_kernel<float, FWD, false> : fft_multi_kernel<double, FWD, false>;
+  launch_kernel(kern, nblk, kThreads, 0, s, a);
+  SHT_HIP(hipGetLastError());
+  return SHT_OK;
+}
+
 }  // namespace
+
+int launch_fft_inv_multi(const MultiGroup *g, int n, hipStream_t s) { return multi_launch<false>(g, n, s); }
+int launch_fft_fwd_multi(const MultiGroup *g, int n, hipStream_t s) { return multi_launch<true>(g, n, s); }
 
 template <int L>
 void capacities(int device, int (&out)[2]) {

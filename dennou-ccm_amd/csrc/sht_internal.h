@@ -310,6 +310,45 @@ int launch_leg_fwd_mixed_shape(const Plan &p, int shape, const float *four, doub
                                hipStream_t s);
 int launch_leg_fwd_mixed(const Plan &p, const float *four, double *spec, int nf, hipStream_t s);
 
+// One launch per stage over several groups of fields on different grids (the
+// ensemble batches): workgroup ranges of one grid each, the same items as the
+// groups' own launches (Legendre: workgroup per (m, 16 columns); FFT: the big
+// blocks), so the results are bitwise theirs.  A group takes part if its grid
+// has at most 64 latitude pairs and 256 longitudes (multi_available); a launch
+// holds at most kMaxMulti groups of one precision form.
+constexpr int kMaxMulti = 8;
+struct MultiGroup {
+  const Plan *p;
+  const double *spec_in;
+  double *grid, *spec_out;
+  int nf;
+};
+bool multi_available(const Plan &p, int nf);
+int launch_leg_inv_f64_multi(const MultiGroup *g, int n, hipStream_t s);
+int launch_leg_fwd_f64_multi(const MultiGroup *g, int n, hipStream_t s);
+int launch_leg_inv_mixed_multi(const MultiGroup *g, int n, hipStream_t s);
+int launch_leg_fwd_mixed_multi(const MultiGroup *g, int n, hipStream_t s);
+int launch_fft_inv_multi(const MultiGroup *g, int n, hipStream_t s);
+int launch_fft_fwd_multi(const MultiGroup *g, int n, hipStream_t s);
+// the intermediate's layout in these launches, whatever the group's size
+inline FourGeom multi_geom(const Plan &p, int nf) { return four_geom_g(p, fft_group(p.im), nf); }
+// non-temporal stores of the intermediate (four_geom_out) for all groups together
+inline bool multi_streams(const MultiGroup *g, int n) {
+  size_t bytes = 0;
+  for (int i = 0; i < n; ++i) {
+    const FourGeom f = multi_geom(*g[i].p, g[i].nf);
+    bytes += (size_t)f.P2 * f.nfg * f.M1 * 2 * ((size_t)1 << f.lg) * (g[i].p->prec == SHT_PREC_FP64 ? 8 : 4);
+  }
+  return bytes <= kStreamFourBytes;
+}
+// index of the group whose workgroups [g[i].blk0, g[i + 1].blk0) hold block b
+template <class Args>
+__device__ __forceinline__ int multi_group(const Args &a, int b) {
+  int i = 0;
+  while (i + 1 < a.ng && b >= a.g[i + 1].blk0) ++i;
+  return i;
+}
+
 // Allocation-free spectral -> grid (sht_noalloc.hip): the static scratch's
 // device address is looked up once per device at plan creation.
 int noalloc_init_device(int device);

@@ -785,13 +785,9 @@ struct StagedUnit {
 
 // Forward, workgroup = (m, CT column tiles); LDS [CT][parity][P2p pairs][16].
 template <int CT, int D, int NW>
-__global__ __launch_bounds__(NW * 64) void leg_fwd_f64_staged_kernel(
-    const double *__restrict__ four, double *__restrict__ spec, const double *__restrict__ Pfwd,
-    const int *__restrict__ poff, const int *__restrict__ mlist, int mlen, int N, int P2, int P2p,
-    int ncol, int nct, FourGeom geo) {
-  extern __shared__ double sb[];
-  int m, t;
-  if (!xcd_m_block(blockIdx.x, mlist, mlen, (nct + CT - 1) / CT, m, t)) return;
+__device__ __forceinline__ void leg_fwd_f64_staged_item(
+    double *sb, const double *__restrict__ four, double *__restrict__ spec, const double *__restrict__ Pfwd,
+    const int *__restrict__ poff, int N, int P2, int P2p, int ncol, FourGeom geo, int m, int t) {
   const int ct0 = t * CT;
   const int wave = wave_id(), lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
   const int nn = N - m + 1, ke = (nn + 1) >> 1, ko = nn >> 1;
@@ -831,20 +827,25 @@ __global__ __launch_bounds__(NW * 64) void leg_fwd_f64_staged_kernel(
   }
 }
 
+template <int CT, int D, int NW>
+__global__ __launch_bounds__(NW * 64) void leg_fwd_f64_staged_kernel(
+    const double *__restrict__ four, double *__restrict__ spec, const double *__restrict__ Pfwd,
+    const int *__restrict__ poff, const int *__restrict__ mlist, int mlen, int N, int P2, int P2p,
+    int ncol, int nct, FourGeom geo) {
+  extern __shared__ double sb[];
+  int m, t;
+  if (!xcd_m_block(blockIdx.x, mlist, mlen, (nct + CT - 1) / CT, m, t)) return;
+  leg_fwd_f64_staged_item<CT, D, NW>(sb, four, spec, Pfwd, poff, N, P2, P2p, ncol, geo, m, t);
+}
+
 // Inverse, workgroup = (m, table, CT column tiles); LDS [CT][parity][KP][16]
 // with KP = this m's degrees per parity rounded up to 4 (rows past a parity's
 // last degree hold zeros).
 template <int CT, int D, int NW, bool NT>
-__global__ __launch_bounds__(NW * 64) void leg_inv_f64_staged_kernel(
-    const double *__restrict__ spec, double *__restrict__ four, double *__restrict__ four2,
-    const double *__restrict__ Pinv, const double *__restrict__ Hinv, const int *__restrict__ poff,
-    const int *__restrict__ mlist, int mlen, int N, int P2, int P2p, int ncol, int nct, int tab0,
-    int ntab, FourGeom geo) {
-  extern __shared__ double sb[];
-  const int ncg = (nct + CT - 1) / CT;
-  int m, t;
-  if (!xcd_m_block(blockIdx.x, mlist, mlen, ntab * ncg, m, t)) return;
-  const int tab = tab0 + t % ntab, ct0 = (t / ntab) * CT;
+__device__ __forceinline__ void leg_inv_f64_staged_item(
+    double *sb, const double *__restrict__ spec, double *__restrict__ four, double *__restrict__ four2,
+    const double *__restrict__ Pinv, const double *__restrict__ Hinv, const int *__restrict__ poff, int N, int P2,
+    int P2p, int ncol, FourGeom geo, int m, int tab, int ct0) {
   const int nn = N - m + 1, ke = (nn + 1) >> 1, ko = nn >> 1;
   const int KP = (ke + 3) & ~3;
   const double *__restrict__ sp = spec + (size_t)coef_off(N, m) * ncol;
@@ -888,12 +889,61 @@ __global__ __launch_bounds__(NW * 64) void leg_inv_f64_staged_kernel(
   }
 }
 
+template <int CT, int D, int NW, bool NT>
+__global__ __launch_bounds__(NW * 64) void leg_inv_f64_staged_kernel(
+    const double *__restrict__ spec, double *__restrict__ four, double *__restrict__ four2,
+    const double *__restrict__ Pinv, const double *__restrict__ Hinv, const int *__restrict__ poff,
+    const int *__restrict__ mlist, int mlen, int N, int P2, int P2p, int ncol, int nct, int tab0,
+    int ntab, FourGeom geo) {
+  extern __shared__ double sb[];
+  const int ncg = (nct + CT - 1) / CT;
+  int m, t;
+  if (!xcd_m_block(blockIdx.x, mlist, mlen, ntab * ncg, m, t)) return;
+  leg_inv_f64_staged_item<CT, D, NW, NT>(sb, spec, four, four2, Pinv, Hinv, poff, N, P2, P2p, ncol, geo, m,
+                                         tab0 + t % ntab, (t / ntab) * CT);
+}
+
+// ---- Several groups in one launch (sht_internal.h, MultiGroup): the staged
+// shape with one column tile and four waves, workgroup ranges per group.
+struct F64Multi {
+  int ng;
+  struct Group {
+    const double *spec_in;
+    double *four, *spec_out;
+    const double *table;
+    const int *poff, *mlist;
+    int blk0, mlen, N, P2, P2p, ncol, nct;
+    FourGeom geo;
+  } g[kMaxMulti];
+};
+
+template <bool FWD, bool NT>
+__global__ __launch_bounds__(256) void leg_f64_multi_kernel(F64Multi a) {
+  extern __shared__ double sb[];
+  const F64Multi::Group &g = a.g[multi_group(a, blockIdx.x)];
+  int m, t;
+  if (!xcd_m_block(blockIdx.x - g.blk0, g.mlist, g.mlen, g.nct, m, t)) return;
+  if constexpr (FWD)
+    leg_fwd_f64_staged_item<1, 4, 4>(sb, g.four, g.spec_out, g.table, g.poff, g.N, g.P2, g.P2p, g.ncol, g.geo, m, t);
+  else
+    leg_inv_f64_staged_item<1, 4, 4, NT>(sb, g.spec_in, g.four, nullptr, g.table, nullptr, g.poff, g.N, g.P2, g.P2p,
+                                         g.ncol, g.geo, m, 0, t);
+}
+
+inline size_t fwd_staged_lds(const Plan &p, int ct) {
+  return sizeof(double) * ct * 2 * p.P2p * 16;  // <= 64 KB: P2p <= 256
+}
+inline size_t inv_staged_lds(const Plan &p, int ct) {
+  // the last tile's rows filled up to a chunk of 16; <= 64 KB: kp0 <= 128
+  const int kp0 = roundup(ceil_half(p.N + 1), 4);
+  return sizeof(double) * ((ct * 2 - 1) * kp0 + roundup(kp0, 16)) * 16;
+}
+
 template <int CT, int NW>
 int fwd_staged_launch(const Plan &p, const double *four, double *spec, int nf, hipStream_t s) {
   const int ncol = 2 * nf, nct = (ncol + 15) / 16;
-  const size_t lds = sizeof(double) * CT * 2 * p.P2p * 16;  // <= 64 KB: P2p <= 256
-  launch_kernel(leg_fwd_f64_staged_kernel<CT, 4, NW>, xcd_m_blocks(p, 1, (nct + CT - 1) / CT), NW * 64, lds,
-      s, four, spec, p.Pfwd, p.poff_fwd, p.xcd_m[1], p.xcd_mlen[1], p.N, p.P2, p.P2p, ncol, nct,
+  launch_kernel(leg_fwd_f64_staged_kernel<CT, 4, NW>, xcd_m_blocks(p, 1, (nct + CT - 1) / CT), NW * 64,
+      fwd_staged_lds(p, CT), s, four, spec, p.Pfwd, p.poff_fwd, p.xcd_m[1], p.xcd_mlen[1], p.N, p.P2, p.P2p, ncol, nct,
       four_geom(p, nf));
   SHT_HIP(hipGetLastError());
   return SHT_OK;
@@ -903,13 +953,10 @@ template <int CT, int NW>
 int inv_staged_launch(const Plan &p, const double *spec, double *four, double *four2, int tab0,
                       int ntab, int nf, hipStream_t s) {
   const int ncol = 2 * nf, nct = (ncol + 15) / 16;
-  const int kp0 = roundup(ceil_half(p.N + 1), 4);
-  // the last tile's rows filled up to a chunk of 16; <= 64 KB: kp0 <= 128
-  const size_t lds = sizeof(double) * ((CT * 2 - 1) * kp0 + roundup(kp0, 16)) * 16;
   const FourGeom geo = four_geom_out(p, nf, sizeof(double));
   launch_kernel(geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true>
                            : leg_inv_f64_staged_kernel<CT, 4, NW, false>,
-      xcd_m_blocks(p, 0, ntab * ((nct + CT - 1) / CT)), NW * 64, lds, s, spec, four, four2, p.Pinv, p.Hinv,
+      xcd_m_blocks(p, 0, ntab * ((nct + CT - 1) / CT)), NW * 64, inv_staged_lds(p, CT), s, spec, four, four2, p.Pinv, p.Hinv,
       p.poff_inv, p.xcd_m[0], p.xcd_mlen[0], p.N, p.P2, p.P2p, ncol, nct, tab0, ntab, geo);
   SHT_HIP(hipGetLastError());
   return SHT_OK;
@@ -1145,6 +1192,28 @@ int fwd_div_launch(const Plan &p, const double *fa, const double *fb, double *sp
   return SHT_OK;
 }
 
+template <bool FWD>
+int f64_multi_launch(const MultiGroup *g, int n, hipStream_t s) {
+  F64Multi a{};
+  a.ng = n;
+  int nblk = 0;
+  size_t lds = 0;
+  for (int i = 0; i < n; ++i) {
+    const Plan &p = *g[i].p;
+    const int ncol = 2 * g[i].nf, nct = (ncol + 15) / 16;
+    a.g[i] = {g[i].spec_in, p.four, g[i].spec_out, FWD ? p.Pfwd : p.Pinv, FWD ? p.poff_fwd : p.poff_inv, p.xcd_m[FWD],
+              nblk, p.xcd_mlen[FWD], p.N, p.P2, p.P2p, ncol, nct, multi_geom(p, g[i].nf)};
+    nblk += xcd_m_blocks(p, FWD, nct);
+    const size_t need = FWD ? fwd_staged_lds(p, 1) : inv_staged_lds(p, 1);
+    lds = need > lds ? need : lds;
+  }
+  launch_kernel(FWD ? leg_f64_multi_kernel<FWD, false>
+                    : (multi_streams(g, n) ? leg_f64_multi_kernel<FWD, true> : leg_f64_multi_kernel<FWD, false>),
+                nblk, 256, lds, s, a);
+  SHT_HIP(hipGetLastError());
+  return SHT_OK;
+}
+
 // Field count from which the staged shape runs in two parts on the T170 grid.
 constexpr int kHalvesMinFields = 192;
 
@@ -1348,6 +1417,18 @@ int launch_leg_fwd_f64_div(const Plan &p, const double *fa, const double *fb, do
   if (p.P2p >= 128 || units > 8)  // 16 P2p <= 4096 column pairs a block, 512 threads
     return p.P2p <= 128 ? fwd_div_launch<8, 4>(p, fa, fb, spec, nf, s) : fwd_div_launch<8, 8>(p, fa, fb, spec, nf, s);
   return p.P2p <= 64 ? fwd_div_launch<4, 4>(p, fa, fb, spec, nf, s) : fwd_div_launch<4, 7>(p, fa, fb, spec, nf, s);
+}
+
+int launch_leg_inv_f64_multi(const MultiGroup *g, int n, hipStream_t s) { return f64_multi_launch<false>(g, n, s); }
+int launch_leg_fwd_f64_multi(const MultiGroup *g, int n, hipStream_t s) { return f64_multi_launch<true>(g, n, s); }
+
+// FP64: a group takes part where its shapes run the staged shape's MFMA
+// sequence (WAVE, TILE and STAGED); the mixed forms' shapes all agree.
+bool multi_available(const Plan &p, int nf) {
+  if (p.P2p > 64 || p.im > 256) return false;
+  if (p.prec != SHT_PREC_FP64) return true;
+  auto same = [](int s) { return s == SHT_SHAPE_WAVE || s == SHT_SHAPE_TILE || s == SHT_SHAPE_STAGED; };
+  return same(resolve_shape(p, nf, 0)) && same(resolve_shape(p, nf, 1));
 }
 
 int launch_leg_inv_f64(const Plan &p, const double *spec, double *four, double *four2,

@@ -672,18 +672,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i
 // units w, w+NW, ... and runs each against every column tile with the same
 // table fragments.  NSL = P2p32 / 32 exactly (the dispatch picks it from the
 // plan).
+template <int MODE, int NSL, int CT>
+struct FwdItemLds {
+  static constexpr size_t bt = sizeof(uint16_t) * CT * 2 * NSL * Form<MODE>::NP * 16 * kRowPitch;
+  static constexpr size_t ebits = Form<MODE>::kScaled ? sizeof(int) * CT * 2 * NSL * 16 : 0;
+  static constexpr size_t bytes = bt + ebits;
+};
+
 template <int MODE, int NSL, int CT, int NW>
-__global__ __launch_bounds__(NW * 64) void leg_fwd_mixed_kernel(
-    const float *__restrict__ four, double *__restrict__ spec, const uint16_t *__restrict__ L,
-    const int *__restrict__ loff, const int *__restrict__ lexp, const int *__restrict__ mlist,
-    int mlen, int N, int P2, int P2p32, int ncol, int nct, FourGeom geo) {
+__device__ __forceinline__ void leg_fwd_mixed_item(
+    unsigned char *lds, const float *__restrict__ four, double *__restrict__ spec, const uint16_t *__restrict__ L,
+    const int *__restrict__ loff, const int *__restrict__ lexp, int N, int P2, int P2p32, int ncol, int nct,
+    FourGeom geo, int m, int t, int tid) {
   constexpr int NP = Form<MODE>::NP, NG = 2 * NSL;  // LDS groups per column tile
-  __shared__ __align__(16) uint16_t bt[CT * NG * NP * 16 * kRowPitch];
-  __shared__ int ebits[CT * NG * 16];
-  int m, t;
-  if (!xcd_m_block(blockIdx.x, mlist, mlen, (nct + CT - 1) / CT, m, t)) return;
+  uint16_t *bt = reinterpret_cast<uint16_t *>(lds);
+  int *ebits = reinterpret_cast<int *>(lds + FwdItemLds<MODE, NSL, CT>::bt);
   const int ct0 = t * CT, nc = nct - ct0 < CT ? nct - ct0 : CT;
-  const int wave = wave_id(), lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, kq = lane >> 4;
   const int nn = N - m + 1, ke = (nn + 1) >> 1;
   const int KR = (ke + 15) & ~15, nrt = KR >> 4;
   double *__restrict__ sm = spec + (size_t)coef_off(N, m) * ncol + ct0 * 16;
@@ -707,7 +712,7 @@ __global__ __launch_bounds__(NW * 64) void leg_fwd_mixed_kernel(
     const bool v = p < P2 && cc < ncol;
     const float x = four[geo.at(v ? p : 0, m, par, v ? cc : ct0 * 16)];
     return v ? x : 0.0f;
-  }, threadIdx.x);
+  }, tid);
   __syncthreads();
   for (int u = wave; u < nunits; u += NW) {
     const int par = u / nrt, rt = u % nrt;
@@ -741,6 +746,84 @@ __global__ __launch_bounds__(NW * 64) void leg_fwd_mixed_kernel(
       }
     }
   }
+}
+
+template <int MODE, int NSL, int CT, int NW>
+__global__ __launch_bounds__(NW * 64) void leg_fwd_mixed_kernel(
+    const float *__restrict__ four, double *__restrict__ spec, const uint16_t *__restrict__ L,
+    const int *__restrict__ loff, const int *__restrict__ lexp, const int *__restrict__ mlist,
+    int mlen, int N, int P2, int P2p32, int ncol, int nct, FourGeom geo) {
+  __shared__ __align__(16) unsigned char lds[FwdItemLds<MODE, NSL, CT>::bytes];
+  int m, t;
+  if (!xcd_m_block(blockIdx.x, mlist, mlen, (nct + CT - 1) / CT, m, t)) return;
+  leg_fwd_mixed_item<MODE, NSL, CT, NW>(lds, four, spec, L, loff, lexp, N, P2, P2p32, ncol, nct, geo, m, t,
+                                        threadIdx.x);
+}
+
+// ---- Several groups in one launch (sht_internal.h, MultiGroup): the KSPLIT
+// items of groups with at most two K slices either way (P2p <= 64, N <= 127).
+struct MixedMulti {
+  int ng;
+  struct Group {
+    const double *spec_in;
+    float *four;
+    double *spec_out;
+    const uint16_t *L;
+    const int *loff, *lexp, *mlist;
+    int blk0, mlen, N, P2, P2p, ncol, nct, nsl;
+    FourGeom geo;
+  } g[kMaxMulti];
+};
+
+template <int MODE, bool NT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void leg_inv_mixed_multi_kernel(MixedMulti a) {
+  __shared__ __align__(16) unsigned char lds[InvItemLds<MODE, 2, 1, 4>::bytes];
+  const MixedMulti::Group &g = a.g[multi_group(a, blockIdx.x)];
+  int m, t;
+  if (!xcd_m_block(blockIdx.x - g.blk0, g.mlist, g.mlen, g.nct, m, t)) return;
+  if (g.nsl == 1)
+    leg_inv_mixed_item<MODE, 1, 1, NT, 4, false>(lds, g.spec_in, g.four, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol,
+                                                 g.nct, g.geo, m, t, threadIdx.x);
+  else
+    leg_inv_mixed_item<MODE, 2, 1, NT, 4, false>(lds, g.spec_in, g.four, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol,
+                                                 g.nct, g.geo, m, t, threadIdx.x);
+}
+
+template <int MODE>
+__global__ __launch_bounds__(256) void leg_fwd_mixed_multi_kernel(MixedMulti a) {
+  __shared__ __align__(16) unsigned char lds[FwdItemLds<MODE, 2, 1>::bytes];
+  const MixedMulti::Group &g = a.g[multi_group(a, blockIdx.x)];
+  int m, t;
+  if (!xcd_m_block(blockIdx.x - g.blk0, g.mlist, g.mlen, g.nct, m, t)) return;
+  if (g.nsl == 1)
+    leg_fwd_mixed_item<MODE, 1, 1, 4>(lds, g.four, g.spec_out, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol, g.nct,
+                                      g.geo, m, t, threadIdx.x);
+  else
+    leg_fwd_mixed_item<MODE, 2, 1, 4>(lds, g.four, g.spec_out, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol, g.nct,
+                                      g.geo, m, t, threadIdx.x);
+}
+
+template <int MODE, bool FWD>
+int mixed_multi_launch(const MultiGroup *g, int n, hipStream_t s) {
+  MixedMulti a{};
+  a.ng = n;
+  int nblk = 0;
+  for (int i = 0; i < n; ++i) {
+    const Plan &p = *g[i].p;
+    const int ncol = 2 * g[i].nf, nct = (ncol + 15) / 16, P2p32 = roundup(p.P2p, 32);
+    a.g[i] = {g[i].spec_in, reinterpret_cast<float *>(p.four), g[i].spec_out,
+              static_cast<const uint16_t *>(FWD ? p.Lfwd : p.Linv), FWD ? p.loff_fwd : p.loff_inv,
+              FWD ? p.lexp_fwd : p.lexp_inv, p.xcd_m[FWD], nblk, p.xcd_mlen[FWD], p.N, p.P2, FWD ? P2p32 : p.P2p,
+              ncol, nct, FWD ? P2p32 / 32 : roundup(ceil_half(p.N + 1), 32) / 32, multi_geom(p, g[i].nf)};
+    nblk += xcd_m_blocks(p, FWD, nct);
+  }
+  if (FWD)
+    launch_kernel(leg_fwd_mixed_multi_kernel<MODE>, nblk, 256, 0, s, a);
+  else
+    launch_kernel(multi_streams(g, n) ? leg_inv_mixed_multi_kernel<MODE, true> : leg_inv_mixed_multi_kernel<MODE, false>,
+                  nblk, 256, 0, s, a);
+  SHT_HIP(hipGetLastError());
+  return SHT_OK;
 }
 
 // Wave shape: each wave owns one 16-column tile of an m and holds that tile's
@@ -1300,6 +1383,24 @@ int launch_leg_fwd_mixed_shape(const Plan &p, int shape, const float *four, doub
 
 int launch_leg_inv_mixed(const Plan &p, const double *spec, float *four, int nf, hipStream_t s) {
   return launch_leg_inv_mixed_shape(p, resolve_shape(p, nf, 0), spec, four, nf, s);
+}
+
+int launch_leg_inv_mixed_multi(const MultiGroup *g, int n, hipStream_t s) {
+  switch (g[0].p->prec) {
+    case SHT_PREC_SPLIT_BF16: return mixed_multi_launch<SHT_PREC_SPLIT_BF16, false>(g, n, s);
+    case SHT_PREC_SCALED_FP16: return mixed_multi_launch<SHT_PREC_SCALED_FP16, false>(g, n, s);
+    case SHT_PREC_SPLIT_BF16X6: return mixed_multi_launch<SHT_PREC_SPLIT_BF16X6, false>(g, n, s);
+  }
+  return fail(SHT_ERR_INVALID, "launch_leg_inv_mixed_multi: not a mixed-precision plan");
+}
+
+int launch_leg_fwd_mixed_multi(const MultiGroup *g, int n, hipStream_t s) {
+  switch (g[0].p->prec) {
+    case SHT_PREC_SPLIT_BF16: return mixed_multi_launch<SHT_PREC_SPLIT_BF16, true>(g, n, s);
+    case SHT_PREC_SCALED_FP16: return mixed_multi_launch<SHT_PREC_SCALED_FP16, true>(g, n, s);
+    case SHT_PREC_SPLIT_BF16X6: return mixed_multi_launch<SHT_PREC_SPLIT_BF16X6, true>(g, n, s);
+  }
+  return fail(SHT_ERR_INVALID, "launch_leg_fwd_mixed_multi: not a mixed-precision plan");
 }
 
 bool fused_inv_available(const Plan &p) { return fused_supported(p) && p.fsync && p.fused_blocks >= 8; }

@@ -215,12 +215,13 @@ int sht_restart_write(const char *path, const sht_restart_desc *desc, const doub
 int sht_restart_read(const char *path, const sht_restart_desc *desc, double *time, double *const fields[10]);
 
 /* ---- ensemble batches: many members of uneven truncation and level count
- *      transformed by one hipGraph launch.  There is no SPML counterpart (SPML
+ *      transformed by one call.  There is no SPML counterpart (SPML
  *      holds one global plan); this is the batched form of wa_xya/xya_wa for
  *      ensemble runs.  Members are grouped by grid (nmax, im, jm); each group's
  *      members are consecutive field ranges of one resident batch, so every
- *      kernel launch covers all members of a group, and the groups run as
- *      independent branches of the graph.                                    */
+ *      kernel launch covers all members of a group; groups of at most 64
+ *      latitude pairs and 256 longitudes share one launch per stage, and
+ *      larger ones run beside them as branches of a hipGraph.                */
 typedef struct sht_batch sht_batch;
 typedef struct {
   int nmax, im, jm; /* truncation and grid of the member */
@@ -239,8 +240,9 @@ void sht_batch_destroy(sht_batch *batch);
 int sht_batch_member(const sht_batch *batch, int j, double **spec_in, double **grid,
                      double **spec_out, int *ld);
 /* Runs the direction (INVERSE: spec_in -> grid; FORWARD: grid -> spec_out;
- * ROUNDTRIP: both) for every member with one graph launch on stream.  The
- * graph is captured on the first call of each direction. */
+ * ROUNDTRIP: both) for every member on stream: one launch per stage where all
+ * groups share theirs, else one graph launch.  The graph is captured on the
+ * first call of each direction. */
 int sht_batch_run(sht_batch *batch, int direction, void *stream);
 /* The same work launched kernel by kernel (no graph), for comparison. */
 int sht_batch_run_eager(sht_batch *batch, int direction, void *stream);

@@ -120,3 +120,36 @@ def test_batch_autotune_keeps_results():
         assert rel(g, oracle.Plan(N, im, jm).spec_to_grid(specs[j])) < 1e-12, j
         assert rel(s, specs[j]) < 1e-12, j
     b.close()
+
+
+MANY = [(7, 16, 10, 3), (5, 16, 8, 40), (10, 32, 16, 1), (9, 32, 26, 70), (21, 64, 32, 33), (20, 64, 48, 5),
+        (31, 64, 64, 17), (42, 128, 64, 9), (50, 128, 100, 2), (85, 256, 128, 11), (100, 256, 202, 4), (0, 16, 2, 8)]
+
+
+@pytest.mark.parametrize("prec", [shtamd.PREC_FP64, shtamd.PREC_SPLIT_BF16, shtamd.PREC_SCALED_FP16, shtamd.PREC_SPLIT_BF16X6])
+@pytest.mark.parametrize("count", [2, len(MANY)])
+def test_batch_shared_launches_bitwise(prec, count):
+    """Two grids in one launch per stage, and more than a launch takes beside one
+    of more latitude pairs: each direction bitwise as the member alone."""
+    members = MANY[-count:] if count > 2 else MANY[4:6]
+    b = shtamd.Batch(members, precision=prec)
+    specs = [synth.spectra(N, nf, cfg=5, member=j) for j, (N, _, _, nf) in enumerate(members)]
+    for j, s in enumerate(specs):
+        spec_in, _, _, ld = b.member_ptrs(j)
+        hipmem.put_member_spectra(spec_in, ld, s)
+    for run in (b.run, b.run_eager):
+        run(shtamd.DIR_INVERSE)
+        run(shtamd.DIR_FORWARD)
+        torch.cuda.synchronize()
+        for j, (N, im, jm, nf) in enumerate(members):
+            _, grid, spec_out, ld = b.member_ptrs(j)
+            p = shtamd.Plan(N, im, jm, nf, precision=prec)
+            si = torch.from_numpy(shtamd.spec_to_real(specs[j])).cuda()
+            ga, so = torch.empty((nf, jm, im), dtype=torch.float64, device="cuda"), torch.empty_like(si)
+            p.spec_to_grid(si, ga, nf)
+            p.grid_to_spec(ga, so, nf)
+            torch.cuda.synchronize()
+            assert np.array_equal(hipmem.from_device(grid, (nf, jm, im)), ga.cpu().numpy()), j
+            assert np.array_equal(hipmem.get_member_spectra(spec_out, ld, p.K, nf), shtamd.real_to_spec(so.cpu().numpy())), j
+            p.close()
+    b.close()
