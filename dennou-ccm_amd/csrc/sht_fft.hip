@@ -51,9 +51,9 @@ struct FwdIO {
 // workgroups of the last, partly empty field group evenly over the XCDs (T85,
 // 97 fields: inverse 9.8 -> 9.5 us); otherwise each XCD takes a contiguous
 // range of tiles, which measured ~1 % faster when blocks queue.
-// One tile of the stage (its block of C values, LDS at buf and twl).
+// One tile of the stage (its block of C values, LDS at buf).
 template <int L, typename TF, bool DIRECT, int C>
-__device__ __forceinline__ void fft_fwd_tile(double2 *buf, double2 *twl, const double *__restrict__ grid,
+__device__ __forceinline__ void fft_fwd_tile(double2 *buf, const double *__restrict__ grid,
                                              TF *__restrict__ four, int mode, const double2 *__restrict__ tw,
                                              const double *__restrict__ coslat, int P2, int M1, int nf, int jm,
                                              int tile, int tid) {
@@ -64,9 +64,8 @@ __device__ __forceinline__ void fft_fwd_tile(double2 *buf, double2 *twl, const d
   const int jn = P2 + p, js = P2 - 1 - p;
   // the twiddles are loaded after the first ring loads are issued (one wait
   // covers both; loaded first, their wait held back every ring load)
-  auto twiddles = [&] {
-    for (int q = tid; q < L; q += kThreads) twl[q] = tw[q];
-  };
+  FftTw<L, C> ft_tw;
+  auto twiddles = [&] { ft_tw.load(tw, tid); };
   // z = f_N + i f_S; transforms past nf are zero
   auto ring = [&](int g, int i) {
     const int f = f0 + g;
@@ -77,11 +76,14 @@ __device__ __forceinline__ void fft_fwd_tile(double2 *buf, double2 *twl, const d
     }
     return z;
   };
-  auto keep = [&](int g, int i, double2 v) {
-    if (i < M1 || i > L - M1) buf[px<L>(g * L + i)] = v;
+  auto keep = [&](int g, int d0, int c, double2 v) {
+    const int i = d0 + c;
+    if (i < M1 || i > L - M1) buf[swz<L>(g * L + d0) ^ swz<L>(c)] = v;
   };
+  auto ring_at = [&](int g, int j, int c) { return ring(g, j + c); };
+  auto staged = [&](int g, int j, int c) { return buf[swz<L>(g * L + j) ^ swz<L>(c)]; };
   if constexpr (DIRECT) {
-    fft_lds<L, -1, C>(buf, twl, ring, keep, tid, twiddles);
+    fft_lds<L, -1, C>(buf, ft_tw, ring_at, keep, tid, twiddles);
   } else {
     constexpr int NQ = C / kThreads;  // samples per thread
     double2 z[NQ];
@@ -92,16 +94,16 @@ __device__ __forceinline__ void fft_fwd_tile(double2 *buf, double2 *twl, const d
     }
     twiddles();
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) buf[px<L>(tid + q * kThreads)] = z[q];
+    for (int q = 0; q < NQ; ++q) buf[swz<L>(tid + q * kThreads)] = z[q];
     __syncthreads();
-    fft_lds<L, -1, C>(buf, twl, [&](int g, int i) { return buf[px<L>(g * L + i)]; }, keep, tid);
+    fft_lds<L, -1, C>(buf, ft_tw, staged, keep, tid);
   }
   const double sc = 0.5 / L * (mode == 0 ? 1.0 : 1.0 / coslat[jn]);
   for (int idx = tid; idx < M1 * G; idx += kThreads) {
     const int m = idx / G, g = idx % G, f = f0 + g;
     if (f >= nf) continue;
-    const double2 zm = buf[px<L>(g * L + m)];
-    const double2 zc = buf[px<L>(g * L + ((L - m) & (L - 1)))];
+    const double2 zm = buf[swz<L>(g * L + m)];
+    const double2 zc = buf[swz<L>(g * L + ((L - m) & (L - 1)))];
     // X_N = (Z_m + conj Z_{L-m}) sc ;  X_S = -i (Z_m - conj Z_{L-m}) sc
     const double2 xn = make_double2((zm.x + zc.x) * sc, (zm.y - zc.y) * sc);
     const double2 xs = make_double2((zm.y + zc.y) * sc, -(zm.x - zc.x) * sc);
@@ -122,11 +124,10 @@ __global__ __launch_bounds__(kThreadsOf<C>) void fft_fwd_kernel(FwdIO<TF> io,
                                                                 const double2 *__restrict__ tw,
                                                                 const double *__restrict__ coslat,
                                                                 int P2, int M1, int nf, int jm, int spread) {
-  __shared__ double2 buf[kPaddedOf<C>];
-  __shared__ double2 twl[L];
+  __shared__ double2 buf[C];
   const int tile = spread ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
   const int sel = blockIdx.y;
-  fft_fwd_tile<L, TF, DIRECT, C>(buf, twl, io.src[sel], io.dst[sel], io.mode[sel], tw, coslat, P2, M1, nf, jm, tile,
+  fft_fwd_tile<L, TF, DIRECT, C>(buf, io.src[sel], io.dst[sel], io.mode[sel], tw, coslat, P2, M1, nf, jm, tile,
                                  threadIdx.x);
 }
 
@@ -145,11 +146,10 @@ __global__ __launch_bounds__(kThreadsOf<C>) void fft_inv_kernel(InvOutputs<TF> i
                                                                 const double2 *__restrict__ tw,
                                                                 const double *__restrict__ coslat,
                                                                 int P2, int M1, int nf, int jm, int spread) {
-  __shared__ double2 buf[kPaddedOf<C>];
-  __shared__ double2 twl[L];
+  __shared__ double2 buf[C];
   const int tile = spread ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
   const int sel = blockIdx.y;
-  fft_inv_tile<L, TF, false, C>(buf, twl, tw, io.src[sel], io.dst[sel], io.mode[sel], coslat, P2, M1, nf, jm,
+  fft_inv_tile<L, TF, false, C>(buf, tw, io.src[sel], io.dst[sel], io.mode[sel], coslat, P2, M1, nf, jm,
                                 tile, threadIdx.x);
 }
 
@@ -179,7 +179,12 @@ int fwd_resident(int device) {
                                                    0) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
     return 0;
-  return per_cu * ncu;
+  // the query counts LDS in bytes; the hardware hands it out in 128ths of a
+  // CU's 160 KB, so of the five 32 KB blocks it names four fit (a launch's time
+  // steps up from 1024 to 1088 blocks on 256 CUs)
+  constexpr int kLdsUnit = 160 * 1024 / 128;
+  const int fit = 128 / ((int)(sizeof(double2) * C + kLdsUnit - 1) / kLdsUnit);
+  return (per_cu < fit ? per_cu : fit) * ncu;
 }
 
 template <int L, int C, typename TF>
@@ -239,10 +244,9 @@ int inv_typed(const Plan &p, const TF *four, const TF *four2, double *grid, doub
 }
 
 // ---- Several groups in one launch (sht_internal.h, MultiGroup): big blocks
-// only, at most kMultiMaxIm longitudes.  Each group's range of workgroups is
+// only, at most 256 longitudes.  Each group's range of workgroups is
 // padded to a multiple of 8, so that its tiles meet the XCDs as in a launch of
 // their own.
-constexpr int kMultiMaxIm = 256;
 struct FftMulti {
   int ng, spread;
   struct Group {
@@ -255,30 +259,29 @@ struct FftMulti {
 };
 
 template <int L, typename TF, bool FWD, bool DIRECT>
-__device__ __forceinline__ void fft_multi_tile(double2 *buf, double2 *twl, const FftMulti::Group &g, int tile) {
+__device__ __forceinline__ void fft_multi_tile(double2 *buf, const FftMulti::Group &g, int tile) {
   TF *four = static_cast<TF *>(const_cast<void *>(g.four));
   if constexpr (FWD)
-    fft_fwd_tile<L, TF, DIRECT, kFftBig>(buf, twl, g.grid, four, 0, g.tw, g.coslat, g.P2, g.M1, g.nf, g.jm, tile,
+    fft_fwd_tile<L, TF, DIRECT, kFftBig>(buf, g.grid, four, 0, g.tw, g.coslat, g.P2, g.M1, g.nf, g.jm, tile,
                                          threadIdx.x);
   else
-    fft_inv_tile<L, TF, false, kFftBig>(buf, twl, g.tw, four, g.grid, 0, g.coslat, g.P2, g.M1, g.nf, g.jm, tile,
+    fft_inv_tile<L, TF, false, kFftBig>(buf, g.tw, four, g.grid, 0, g.coslat, g.P2, g.M1, g.nf, g.jm, tile,
                                         threadIdx.x);
 }
 
 template <typename TF, bool FWD, bool DIRECT>
 __global__ __launch_bounds__(kThreads) void fft_multi_kernel(FftMulti a) {
-  __shared__ double2 buf[kLdsPadded];
-  __shared__ double2 twl[kMultiMaxIm];
+  __shared__ double2 buf[kLdsComplex];
   const FftMulti::Group &g = a.g[multi_group(a, blockIdx.x)];
   const int b = blockIdx.x - g.blk0;
   if (b >= g.nblk) return;
   const int tile = a.spread ? b : xcd_tile(b, g.nblk);
   switch (g.im) {
-    case 16: return fft_multi_tile<16, TF, FWD, DIRECT>(buf, twl, g, tile);
-    case 32: return fft_multi_tile<32, TF, FWD, DIRECT>(buf, twl, g, tile);
-    case 64: return fft_multi_tile<64, TF, FWD, DIRECT>(buf, twl, g, tile);
-    case 128: return fft_multi_tile<128, TF, FWD, DIRECT>(buf, twl, g, tile);
-    case 256: return fft_multi_tile<256, TF, FWD, DIRECT>(buf, twl, g, tile);
+    case 16: return fft_multi_tile<16, TF, FWD, DIRECT>(buf, g, tile);
+    case 32: return fft_multi_tile<32, TF, FWD, DIRECT>(buf, g, tile);
+    case 64: return fft_multi_tile<64, TF, FWD, DIRECT>(buf, g, tile);
+    case 128: return fft_multi_tile<128, TF, FWD, DIRECT>(buf, g, tile);
+    case 256: return fft_multi_tile<256, TF, FWD, DIRECT>(buf, g, tile);
   }
 }
 

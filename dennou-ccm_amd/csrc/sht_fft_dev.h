@@ -23,20 +23,25 @@ namespace {
 // fft_block.
 template <int C>
 constexpr int kThreadsOf = C / 8;
-// LDS holds one pad element per 16 complex values -- the radix-16 pass writes
-// 16 consecutive outputs per thread (a 256-byte lane stride), which without the
-// pad lands every lane of a ds_write on the same banks -- and one more per
-// transform, because the Fourier-side loops run the G transforms of a block in
-// consecutive lanes (element m of transform g), a stride of L(1 + 1/16)
-// elements that is otherwise a multiple of the bank count.
-template <int C>
-constexpr int kPaddedOf = C + C / 16 + C / 16;
+// LDS holds exactly the block's C complex values: element i (i = g L + n of
+// transform g) lies at swz<L>(i), the low four bits XORed with the bits above
+// them.  Without that a radix-16 pass writes at a lane stride of 256 bytes and
+// the Fourier-side loops, which run the transforms of a block in consecutive
+// lanes, at strides of 16 L bytes: one 16-byte bank group each.  The bits of
+// a block's transform index enter one place higher from L = 256 up, where a
+// wave's lanes hold 8 consecutive n of 8 transforms (or more n of fewer).
+// Padding instead (one element per 16 and one per transform) took 36.8 KB a
+// big block, with the twiddles in LDS too 41-45 KB: 3 blocks per CU at 512
+// longitudes, where 32 KB allow 4.  T170 (512 longitudes), inverse / forward:
+// 776 fields FP32 225 / 217 -> 199 / 194 us, 145 fields FP64 54 / 54 -> 46.6 /
+// 47.0; up to 256 longitudes, 4 blocks per CU either way, the times stay.
+// swz is linear in the bits, so for indexes without common bits swz(a + c) =
+// swz(a) ^ swz(c): a butterfly's accesses cost one XOR with a constant each.
+template <int L>
+__device__ __forceinline__ constexpr int swz(int i) { return i ^ ((i >> 4) & 15) ^ (((i >> 8) << (L >= 256 ? 1 : 0)) & 15); }
 // the big block, as the fused inverse uses it
 constexpr int kThreads = kThreadsOf<kFftBig>;
 constexpr int kLdsComplex = kFftBig;
-constexpr int kLdsPadded = kPaddedOf<kFftBig>;
-template <int L>
-__device__ __forceinline__ int px(int i) { return i + (i >> 4) + i / L; }
 
 // Regular stores: the Legendre step that reads the Fourier data next finds
 // them in the Infinity Cache (streaming them made it slower at every size).
@@ -128,22 +133,36 @@ __host__ __device__ inline int four_tiles(int P2, int nf) {
 
 // One Stockham pass of radix R over G transforms of length L, Ns the product
 // of the radices already applied.  Butterfly j of transform g reads
-// x[j + r L/R] (in(g, i) returns element i of transform g), applies
+// x[j + r L/R] (in(g, j, c) returns element j + c of transform g, the bits of c
+// above those of j), applies
 // w^(r k L/(Ns R)) (k = j mod Ns; the powers are built by repeated
-// multiplication from one LDS twiddle), runs a register DFT and writes
-// y[(j/Ns) Ns R + k + r Ns] through out(g, i, v).  A barrier separates the
+// multiplication from one twiddle per butterfly, which the thread holds in
+// registers from the start), runs a register DFT and writes
+// y[(j/Ns) Ns R + k + r Ns] through out(g, i, c, v) (element i + c, no
+// common bits).  A barrier separates the
 // reads from the writes (the passes run in place in buf) and follows them.
 struct NoHook {
   __device__ void operator()() const {}
 };
 
+// Butterflies of one pass in the block and per thread, and a thread's twiddles
+// for them (none for Ns = 1).
+template <int L, int R, int Ns, int C>
+struct PassTw {
+  static constexpr int NB = C / L * (L / R), QB = (NB + kThreadsOf<C> - 1) / kThreadsOf<C>;
+  double2 w[QB];
+  __device__ __forceinline__ void load(const double2 *__restrict__ tw, int tid) {
+    if constexpr (Ns > 1)
+#pragma unroll
+      for (int q = 0; q < QB; ++q) w[q] = tw[((tid + q * kThreadsOf<C>) % (L / R)) % Ns * (L / (Ns * R))];
+  }
+};
+
 template <int L, int R, int Ns, int SIGN, int C, class In, class Out, class Hook = NoHook>
-__device__ __forceinline__ void stockham_pass(const double2 *tw, In in, Out out, int tid, Hook hook = {}) {
+__device__ __forceinline__ void stockham_pass(const PassTw<L, R, Ns, C> &tw, In in, Out out, int tid, Hook hook = {}) {
 #pragma clang fp contract(off)
-  constexpr int G = C / L;
   constexpr int kThreads = kThreadsOf<C>;
-  constexpr int NB = G * (L / R);                       // butterflies in the block
-  constexpr int QB = (NB + kThreads - 1) / kThreads;    // per thread
+  constexpr int NB = PassTw<L, R, Ns, C>::NB, QB = PassTw<L, R, Ns, C>::QB;
   double2 v[QB][R];
   // all of the pass's reads first, then hook() (work whose own loads then
   // share one wait with them), then the butterflies
@@ -153,16 +172,15 @@ __device__ __forceinline__ void stockham_pass(const double2 *tw, In in, Out out,
     if (NB % kThreads != 0 && idx >= NB) continue;
     const int g = idx / (L / R), j = idx % (L / R);
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[q][r] = in(g, j + r * (L / R));
+    for (int r = 0; r < R; ++r) v[q][r] = in(g, j, r * (L / R));
   }
   hook();
 #pragma unroll
   for (int q = 0; q < QB; ++q) {
     const int idx = tid + q * kThreads;
     if (NB % kThreads != 0 && idx >= NB) continue;
-    const int j = idx % (L / R), k = j % Ns;
     if constexpr (Ns > 1) {
-      double2 w1 = tw[k * (L / (Ns * R))];
+      double2 w1 = tw.w[q];
       w1.y *= SIGN;
       double2 w = w1;
 #pragma unroll
@@ -181,53 +199,57 @@ __device__ __forceinline__ void stockham_pass(const double2 *tw, In in, Out out,
     const int g = idx / (L / R), j = idx % (L / R), k = j % Ns;
     const int d0 = (j / Ns) * Ns * R + k;
 #pragma unroll
-    for (int r = 0; r < R; ++r) out(g, d0 + r * Ns, v[q][r]);
+    for (int r = 0; r < R; ++r) out(g, d0, r * Ns, v[q][r]);
   }
   __syncthreads();
 }
 
+// Radix plan: 16 = 16, 32 = 8*4, 64 = 8*8, 128 = 16*8, 256 = 16*16,
+// 512 = 8*8*8, 1024 = 16*16*4, 2048 = 16*16*8: R1 * R2 * R3.
+template <int L>
+struct Radix {
+  static constexpr int R1 = L == 32 || L == 64 || L == 512 ? 8 : 16;
+  static constexpr int R2 = L == 16 ? 1 : L == 32 ? 4 : L == 64 || L == 128 || L == 512 ? 8 : 16;
+  static constexpr int R3 = L / (R1 * R2);
+};
+
+// A thread's twiddles of all passes of one FFT, from the global table tw of
+// e^{+2 pi i t / L}; loaded by the caller beside its first data loads.
+template <int L, int C>
+struct FftTw {
+  PassTw<L, Radix<L>::R1, 1, C> t1;
+  PassTw<L, Radix<L>::R2, Radix<L>::R1, C> t2;
+  PassTw<L, Radix<L>::R3, Radix<L>::R1 * Radix<L>::R2, C> t3;
+  __device__ __forceinline__ void load(const double2 *__restrict__ tw, int tid) {
+    if constexpr (Radix<L>::R2 > 1) t2.load(tw, tid);
+    if constexpr (Radix<L>::R3 > 1) t3.load(tw, tid);
+  }
+};
+
 // Complex FFT of G = C / L transforms, exponent sign SIGN (-1
-// forward, +1 inverse), unnormalised; tw (in LDS) holds e^{+2 pi i t / L}.
-// The first pass reads through first(g, i) and the last writes through
-// last(g, i, v), so a caller can feed the first butterflies straight from
+// forward, +1 inverse), unnormalised.
+// The first pass reads through first(g, i, c) and the last writes through
+// last(g, i, c, v) (element i + c, see stockham_pass), so a caller can feed the first butterflies straight from
 // global memory, skip known zeros, or store the results straight out, and
 // save the LDS round trips; the passes between run in place in buf.
-// Radix plan: 16 = 16, 32 = 8*4, 64 = 8*8, 128 = 16*8, 256 = 16*16,
-// 512 = 8*8*8, 1024 = 16*16*4, 2048 = 16*16*8.  Ends with a barrier.
+// Ends with a barrier.
 // hook() runs in the first pass once its reads are issued (see stockham_pass).
 template <int L, int SIGN, int C, class First, class Last, class Hook = NoHook>
-__device__ __forceinline__ void fft_lds(double2 *buf, const double2 *tw, First first, Last last, int tid,
+__device__ __forceinline__ void fft_lds(double2 *buf, const FftTw<L, C> &tw, First first, Last last, int tid,
                                         Hook hook = {}) {
 #pragma clang fp contract(off)
-  auto rd = [&](int g, int i) { return buf[px<L>(g * L + i)]; };
-  auto wr = [&](int g, int i, double2 v) { buf[px<L>(g * L + i)] = v; };
-  if constexpr (L == 16) {
-    stockham_pass<L, 16, 1, SIGN, C>(tw, first, last, tid, hook);
-  } else if constexpr (L == 32) {
-    stockham_pass<L, 8, 1, SIGN, C>(tw, first, wr, tid, hook);
-    stockham_pass<L, 4, 8, SIGN, C>(tw, rd, last, tid);
-  } else if constexpr (L == 64) {
-    stockham_pass<L, 8, 1, SIGN, C>(tw, first, wr, tid, hook);
-    stockham_pass<L, 8, 8, SIGN, C>(tw, rd, last, tid);
-  } else if constexpr (L == 128) {
-    stockham_pass<L, 16, 1, SIGN, C>(tw, first, wr, tid, hook);
-    stockham_pass<L, 8, 16, SIGN, C>(tw, rd, last, tid);
-  } else if constexpr (L == 256) {
-    stockham_pass<L, 16, 1, SIGN, C>(tw, first, wr, tid, hook);
-    stockham_pass<L, 16, 16, SIGN, C>(tw, rd, last, tid);
-  } else if constexpr (L == 512) {
-    stockham_pass<L, 8, 1, SIGN, C>(tw, first, wr, tid, hook);
-    stockham_pass<L, 8, 8, SIGN, C>(tw, rd, wr, tid);
-    stockham_pass<L, 8, 64, SIGN, C>(tw, rd, last, tid);
-  } else if constexpr (L == 1024) {
-    stockham_pass<L, 16, 1, SIGN, C>(tw, first, wr, tid, hook);
-    stockham_pass<L, 16, 16, SIGN, C>(tw, rd, wr, tid);
-    stockham_pass<L, 4, 256, SIGN, C>(tw, rd, last, tid);
+  constexpr int R1 = Radix<L>::R1, R2 = Radix<L>::R2, R3 = Radix<L>::R3;
+  auto rd = [&](int g, int i, int c) { return buf[swz<L>(g * L + i) ^ swz<L>(c)]; };
+  auto wr = [&](int g, int i, int c, double2 v) { buf[swz<L>(g * L + i) ^ swz<L>(c)] = v; };
+  if constexpr (R2 == 1) {
+    stockham_pass<L, R1, 1, SIGN, C>(tw.t1, first, last, tid, hook);
+  } else if constexpr (R3 == 1) {
+    stockham_pass<L, R1, 1, SIGN, C>(tw.t1, first, wr, tid, hook);
+    stockham_pass<L, R2, R1, SIGN, C>(tw.t2, rd, last, tid);
   } else {
-    static_assert(L == 2048, "unsupported ring length");
-    stockham_pass<L, 16, 1, SIGN, C>(tw, first, wr, tid, hook);
-    stockham_pass<L, 16, 16, SIGN, C>(tw, rd, wr, tid);
-    stockham_pass<L, 8, 256, SIGN, C>(tw, rd, last, tid);
+    stockham_pass<L, R1, 1, SIGN, C>(tw.t1, first, wr, tid, hook);
+    stockham_pass<L, R2, R1, SIGN, C>(tw.t2, rd, wr, tid);
+    stockham_pass<L, R3, R1 * R2, SIGN, C>(tw.t3, rd, last, tid);
   }
 }
 
@@ -263,15 +285,14 @@ __device__ __forceinline__ double2 widen(double2 v) { return v; }
 
 // One inverse tile: four (even/odd Legendre sums) -> grid for latitude pair
 // p and field group fgr (tile = fgr * P2 + p).  A thread's Fourier loads (at
-// most 4 (m, field) pairs: M1 * G <= L/2 * G = C/2) and, with tw not NULL,
-// the twiddles into twl are issued before any LDS traffic (with tw NULL the
-// caller has filled twl and synchronised).  Only the coefficients m < M1 and
+// most 4 (m, field) pairs: M1 * G <= L/2 * G = C/2) and its twiddles' are
+// issued before any LDS traffic.  Only the coefficients m < M1 and
 // L - m are placed in LDS: the first FFT pass takes the band between them as
 // zeros without reading it, and the last pass stores the rings straight to
 // the grid (non-temporal).  mode: 0 value, 1 GradLon (x i m / cos lat),
 // 2 GradLat (x 1 / cos lat).  Ends with a barrier.
 template <int L, typename TF, bool COH, int C = kFftBig>
-__device__ __forceinline__ void fft_inv_tile(double2 *buf, double2 *twl, const double2 *__restrict__ tw,
+__device__ __forceinline__ void fft_inv_tile(double2 *buf, const double2 *__restrict__ tw,
                                              const TF *__restrict__ src, double *__restrict__ dst, int mode,
                                              const double *__restrict__ coslat, int P2, int M1, int nf, int jm,
                                              int tile, int tid) {
@@ -298,8 +319,8 @@ __device__ __forceinline__ void fft_inv_tile(double2 *buf, double2 *twl, const d
     Er[q] = load_four_raw<COH>(e);
     Or[q] = load_four_raw<COH>(e + 2 * FourTile<G>::GL);
   }
-  if (tw)
-    for (int q = tid; q < L; q += kThreads) twl[q] = tw[q];
+  FftTw<L, C> ft_tw;
+  ft_tw.load(tw, tid);
 #pragma unroll
   for (int q = 0; q < NM; ++q) {
     const int idx = tid + q * kThreads;
@@ -316,25 +337,26 @@ __device__ __forceinline__ void fft_inv_tile(double2 *buf, double2 *twl, const d
       xs = make_double2(xs.x * rc, xs.y * rc);
     }
     if (m == 0) {
-      buf[px<L>(g * L)] = make_double2(xn.x, xs.x);
+      buf[swz<L>(g * L)] = make_double2(xn.x, xs.x);
     } else {
-      buf[px<L>(g * L + m)] = make_double2(xn.x - xs.y, xn.y + xs.x);
-      buf[px<L>(g * L + L - m)] = make_double2(xn.x + xs.y, -xn.y + xs.x);
+      buf[swz<L>(g * L + m)] = make_double2(xn.x - xs.y, xn.y + xs.x);
+      buf[swz<L>(g * L + L - m)] = make_double2(xn.x + xs.y, -xn.y + xs.x);
     }
   }
   __syncthreads();
   // transforms past nf hold stale LDS values: their rings are not stored
-  auto spectrum = [&](int g, int i) {
-    return (i < M1 || i > L - M1) ? buf[px<L>(g * L + i)] : make_double2(0.0, 0.0);
+  auto spectrum = [&](int g, int j, int c) {
+    const int i = j + c;
+    return (i < M1 || i > L - M1) ? buf[swz<L>(g * L + j) ^ swz<L>(c)] : make_double2(0.0, 0.0);
   };
-  auto rings = [&](int g, int i, double2 z) {
-    const int f = f0 + g;
+  auto rings = [&](int g, int d0, int c, double2 z) {
+    const int f = f0 + g, i = d0 + c;
     if (f < nf) {
       __builtin_nontemporal_store(z.x, dst + ((size_t)f * jm + jn) * L + i);
       __builtin_nontemporal_store(z.y, dst + ((size_t)f * jm + js) * L + i);
     }
   };
-  fft_lds<L, +1, C>(buf, twl, spectrum, rings, tid);
+  fft_lds<L, +1, C>(buf, ft_tw, spectrum, rings, tid);
 }
 
 }  // namespace

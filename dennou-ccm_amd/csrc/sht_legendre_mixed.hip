@@ -531,9 +531,8 @@ __device__ __forceinline__ int sync_add(int *a, int v) {
 template <int L, int MODE, int NSL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void inv_fused_kernel(FusedInv a) {
   using Lds = InvItemLds<MODE, NSL, 1, 4>;
-  constexpr size_t kFft = sizeof(double2) * kLdsPadded;
+  constexpr size_t kFft = sizeof(double2) * kLdsComplex;
   __shared__ __align__(16) unsigned char lds[Lds::bytes > kFft ? Lds::bytes : kFft];
-  __shared__ double2 twl[L];
   __shared__ int s_item, s_bad;
   constexpr int kDone = -1;
   const int tid = threadIdx.x, x = blockIdx.x & 7;
@@ -543,7 +542,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i
   constexpr int GF = kLdsComplex / L;  // fields per FFT tile
   const int nF = four_tiles<GF>(a.P2, a.nf), nFx = (nF - x + 7) >> 3;
   const int need = a.need;
-  for (int q = tid; q < L; q += 256) twl[q] = a.tw[q];
   // Next item, chosen by thread 0: >= 0 Legendre item (queue << 24 | index),
   // <= -2 FFT tile -2 - tile, kDone.  Thread 0 keeps its queue state.
   bool own_done = false, all_taken = false;
@@ -645,7 +643,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i
       if (tid == 0) sync_add(slot(kFusedSyncHead + t), 1);
     } else {
       const int tile = -2 - item;
-      fft_inv_tile<L, float, true>(reinterpret_cast<double2 *>(lds), twl, nullptr, a.four, a.grid, 0,
+      fft_inv_tile<L, float, true>(reinterpret_cast<double2 *>(lds), a.tw, a.four, a.grid, 0,
                                    a.coslat, a.P2, a.N + 1, a.nf, a.jm, tile, ltid);
       if (bad) {
         constexpr int G = GF;
