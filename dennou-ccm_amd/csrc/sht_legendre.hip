@@ -1309,17 +1309,18 @@ int resolve_shape(const Plan &p, int nf, int dir) {
   // speed alone -- two column tiles per workgroup from 128 latitude pairs
   // (T170: faster in both directions at 97 to 776 fields), one below.  On
   // the 128-pair grid the inverse streams (STAGED): always in the
-  // six-product form, up to 8 fields in the two-piece forms, which run
-  // KSPLIT up to 24 fields.  T170 inverse Legendre step, KSPLIT / TILE /
-  // STAGED, us: x6 9 fields 8.5 / 10.7 / 8.1, 33 fields 15.9 / 14.2 /
-  // 13.6, 97 fields 30.9 / 29.7 / 25.9, 388 fields 107 / 98.8 / 82.7, 776
-  // fields 263 / 234 / 213; BF16 x3 4 fields 6.3 / 6.4 / 4.9, 17 fields
-  // 8.8 / 9.8 / 9.0, 97 fields 23.4 / 21.1 / 21.9, 776 fields 221 / 182 /
-  // 190.  Below 128 pairs the four idle table waves cost more than the
-  // stream saves (T85 x6, 97 fields: KSPLIT 8.3, STAGED 10.1 us).
+  // six-product form, up to 8 fields and from 192 in the two-piece forms, which
+  // run KSPLIT from 9 to 24 fields.  T170 inverse Legendre step, KSPLIT / TILE /
+  // STAGED, us: x6 8 fields 9.4 / 9.3 / 7.2, 33 fields 15.9 / 14.0 / 13.6, 97
+  // fields 31.8 / 29.6 / 25.6, 388 fields 121 / 105 / 86, 776 fields 227 / 197 /
+  // 156; BF16 x3 8 fields 7.5 / 7.6 / 5.5, 17 fields 8.9 / 10.0 / 9.5, 97 fields
+  // 24.3 / 21.8 / 22.1, 250 fields 66 / 56 / 52, 776 fields 177 / 146 / 140;
+  // scaled FP16 97 fields 25.7 / 22.8 / 23.8, 250 fields 70 / 56 / 55, 776
+  // fields 189 / 152 / 145.  Below 128 pairs the idle table waves cost more
+  // than the stream saves (BF16 x3, 100 pairs, 145 fields: 17.3 / 17.7 / 18.0).
   if (p.prec != SHT_PREC_FP64) {
     if (dir == 0 && p.P2p == 128 && mixed_stream_available(p)) {
-      if (p.prec == SHT_PREC_SPLIT_BF16X6 || nf <= 8) return SHT_SHAPE_STAGED;
+      if (p.prec == SHT_PREC_SPLIT_BF16X6 || nf <= 8 || nf >= 192) return SHT_SHAPE_STAGED;
       if (nf <= 24) return SHT_SHAPE_KSPLIT;
     }
     return p.P2p >= 128 ? SHT_SHAPE_TILE : SHT_SHAPE_KSPLIT;

@@ -926,55 +926,58 @@ __global__ __launch_bounds__(256) void leg_inv_mixed_wave_kernel(
   }
 }
 
-// Streaming inverse (shape STAGED of the mixed forms, grids of 128 latitude
-// pairs): the table stays in registers while the data stream past it.
-// Workgroup = (m, a chunk of cs column tiles) of eight waves; wave w holds the
-// table fragments of row tile w for the whole chunk, so each m's table is
-// read once per chunk instead of once per one or two column tiles.  The
-// spectral tiles pass through two LDS buffers: wave w stages group w of each
-// column tile (2 nsl <= 8 groups: parity, K slice) from registers loaded PD
-// tiles ahead.  (The compiler's wait counting has each tile's conversion wait
-// for every earlier load, so fewer tiles stay in flight than issued; forcing
-// exact counts -- the table awaited first, no branch around the loads, the
-// steps unrolled -- measured slower below 776 fields and equal at 776.)
-// Per output tile the products,
-// their order and the stores are those of leg_inv_mixed_item, so the results
-// equal the other shapes' bitwise.  One workgroup per CU (the table takes
-// 72 of the six-product form's ~210 registers at 128 pairs).
+// Streaming inverse (shape STAGED of the mixed forms, grids of at most 128
+// latitude pairs): the table stays in registers while the data stream past it.
+// Workgroup = (m, a chunk of cs column tiles) of sixteen waves; wave w holds
+// the table fragments of row tile w % 8 and parity w / 8 for the whole chunk,
+// so each m's table is read once per chunk instead of once per one or two
+// column tiles.  The spectral tiles pass through two LDS buffers: the waves
+// of one half stage the even tiles, those of the other the odd ones, wave w
+// group w % 8 (2 nsl <= 8 groups: parity, K slice) from registers loaded PD of
+// its tiles ahead.  (The compiler's wait counting has each tile's conversion
+// wait for every earlier load, so fewer tiles stay in flight than issued.)
+// Per output tile the products, their order and the sums are those of
+// leg_inv_mixed_item, so the results equal the other shapes' bitwise.
+// One workgroup per CU: the step is bound by its memory traffic and by how
+// little of the conversions, MFMAs and FP64 sums two waves per SIMD hide
+// behind it, so both parities have waves of their own (four per SIMD).  T170,
+// 776 fields, split-BF16 x6: 156 us against 174 us with eight waves, each
+// holding both parities (72 table registers of ~210).
 template <int MODE, int NSL, bool NT, int PD>
-__global__ __launch_bounds__(512) void leg_inv_mixed_stream_kernel(
+__global__ __launch_bounds__(1024) void leg_inv_mixed_stream_kernel(
     const double *__restrict__ spec, float *__restrict__ four, const uint16_t *__restrict__ L,
     const int *__restrict__ loff, const int *__restrict__ lexp, const int *__restrict__ mlist,
     int mlen, int N, int P2, int P2p, int ncol, int nct, int cs, FourGeom geo) {
-  constexpr int NW = 8, NP = Form<MODE>::NP;
-  using One = InvItemLds<MODE, NSL, 1, NW>;
+  constexpr int NP = Form<MODE>::NP;
+  using One = InvItemLds<MODE, NSL, 1, 1>;
   constexpr size_t kBuf = One::bt + One::ebits;
-  __shared__ __align__(16) unsigned char lds[2 * kBuf + One::obuf];
+  constexpr int kPitch = 20;  // output patch: 16 columns of a pair row, padded
+  __shared__ __align__(16) unsigned char lds[2 * kBuf + sizeof(float) * 16 * 16 * kPitch];
   int m, t;
   if (!xcd_m_block(blockIdx.x, mlist, mlen, (nct + cs - 1) / cs, m, t)) return;
-  const int wave = wave_id(), lane = threadIdx.x & 63, c = lane & 15, k8 = lane >> 4;
+  const int wave = wave_id(), w8 = wave & 7, half = wave >> 3;
+  const int lane = threadIdx.x & 63, c = lane & 15, k8 = lane >> 4;
   const int j0 = t * cs, nj = nct - j0 < cs ? nct - j0 : cs;
   const int nn = N - m + 1, ke = (nn + 1) >> 1, ko = nn >> 1;
   const int KP32 = (ke + 31) & ~31, nsl = KP32 >> 5;
   const double *__restrict__ sm = spec + (size_t)coef_off(N, m) * ncol;
   const uint16_t *__restrict__ Lm = L + loff[m];
-  const bool mma = wave < (P2p >> 4);
-  uint4 pa[2][NSL][3];
+  // this wave's output: row tile w8, parity half
+  const bool mma = w8 < (P2p >> 4);
+  uint4 pa[NSL][3];
   if (mma) {
 #pragma unroll
-    for (int par = 0; par < 2; ++par)
+    for (int s = 0; s < NSL; ++s)
 #pragma unroll
-      for (int s = 0; s < NSL; ++s)
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-          pa[par][s][q] = (q < NP && s < nsl) ? *reinterpret_cast<const uint4 *>(
-                                                    Lm + ((size_t)(par * NP + q) * P2p + wave * 16 + c) * KP32 +
-                                                    s * 32 + k8 * 8)
-                                              : make_uint4(0, 0, 0, 0);
+      for (int q = 0; q < 3; ++q)
+        pa[s][q] = (q < NP && s < nsl) ? *reinterpret_cast<const uint4 *>(
+                                             Lm + ((size_t)(half * NP + q) * P2p + w8 * 16 + c) * KP32 + s * 32 + k8 * 8)
+                                       : make_uint4(0, 0, 0, 0);
   }
-  // this wave's group: parity gpar, K slice gs, LDS slot gpar NSL + gs
-  const bool stg = wave < 2 * nsl;
-  const int gpar = wave >= nsl, gs = wave - gpar * nsl, kend = gpar ? ko : ke;
+  // this wave's staging: tiles j with j % 2 = half, group w8: parity gpar, K
+  // slice gs, LDS slot gpar NSL + gs
+  const bool stg = w8 < 2 * nsl;
+  const int gpar = w8 >= nsl, gs = w8 - gpar * nsl, kend = gpar ? ko : ke;
   auto load = [&](int j, double (&v)[8]) {
     const int col = (j0 + j) * 16 + c;
 #pragma unroll
@@ -985,7 +988,7 @@ __global__ __launch_bounds__(512) void leg_inv_mixed_stream_kernel(
     }
   };
   auto put = [&](int j, const double (&v)[8]) {
-    unsigned char *b = lds + (j & 1) * kBuf;
+    unsigned char *b = lds + half * kBuf;  // j & 1 == half
     const int col = (j0 + j) * 16 + c;
     float f[8];
 #pragma unroll
@@ -1004,31 +1007,48 @@ __global__ __launch_bounds__(512) void leg_inv_mixed_stream_kernel(
     for (int q = 0; q < NP; ++q)
       *reinterpret_cast<uint4 *>(bt + ((size_t)(g * NP + q) * 16 + c) * kRowPitch + k8 * 8) = pc[q];
   };
-  const double ea0 = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m]) : 1.0;
-  const double ea1 = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m + 1]) : 1.0;
-  float *ob = reinterpret_cast<float *>(lds + 2 * kBuf) + wave * (16 * kOutPitch);
-  // column tile j: its staged values in v, convert them, then (barrier) load
-  // tile j + PD into v and multiply tile j
-  auto step = [&](int j, double (&v)[8]) {
-    if (stg) put(j, v);
-    __syncthreads();
-    if (stg && j + PD < nj) load(j + PD, v);
-    if (mma) {
-      const unsigned char *b = lds + (j & 1) * kBuf;
-      inv_tile<MODE, NSL, NT, false>(reinterpret_cast<const uint16_t *>(b), reinterpret_cast<const int *>(b + One::bt),
-                                     ob, pa, ea0, ea1, nsl, four, geo, P2, ncol, m, wave, j0 + j, lane);
+  const double ea = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m + half]) : 1.0;
+  float *ob = reinterpret_cast<float *>(lds + 2 * kBuf) + wave * (16 * kPitch);
+  const int cend = geo.nfg << geo.lg;
+  auto multiply = [&](int j) {
+    const unsigned char *b = lds + (j & 1) * kBuf;
+    const uint16_t *bt = reinterpret_cast<const uint16_t *>(b);
+    const int *ebits = reinterpret_cast<const int *>(b + One::bt);
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < NSL; ++s) {
+      if (s >= nsl) break;
+      const int g = half * NSL + s;
+      uint4 pb[3];
+      load_pb<MODE>(bt, g, k8, c, pb);
+      slice_mac<MODE>(pa[s], pb, Form<MODE>::kScaled ? ea * ldexp(1.0, -ebits[g * 16 + c]) : 1.0, acc);
     }
+    // 4 consecutive columns per lane through the wave's patch [16 pairs][16
+    // columns]; the padding columns of the last field group are written too
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ob[(k8 * 4 + i) * kPitch + c] = (float)acc[i];
+    const int pl = lane >> 2, c4 = (lane & 3) * 4, p = w8 * 16 + pl, cc = (j0 + j) * 16 + c4;
+    const f4 v = *reinterpret_cast<const f4 *>(ob + pl * kPitch + c4);
+    if (p < P2 && cc < cend) put_four<NT>(reinterpret_cast<f4 *>(four + geo.at(p, m, half, cc)), v);
   };
+  // column tile j: the staging half converts its loaded values into buffer j
+  // % 2, then (barrier) loads its tile after the next PD - 1, and all multiply
   double v[PD][8];
   if (stg) {
 #pragma unroll
     for (int d = 0; d < PD; ++d)
-      if (d < nj) load(d, v[d]);
+      if (2 * d + half < nj) load(2 * d + half, v[d]);
   }
-  for (int j = 0; j < nj; j += PD) {
+  for (int j = 0; j < nj; j += 2 * PD) {
 #pragma unroll
-    for (int d = 0; d < PD; ++d)
-      if (j + d < nj) step(j + d, v[d]);
+    for (int d = 0; d < 2 * PD; ++d) {
+      if (j + d >= nj) break;
+      const bool mine = stg && (d & 1) == half;
+      if (mine) put(j + d, v[d / 2]);
+      __syncthreads();
+      if (mine && j + d + 2 * PD < nj) load(j + d + 2 * PD, v[d / 2]);
+      if (mma) multiply(j + d);
+    }
   }
 }
 
@@ -1188,16 +1208,17 @@ int build_mixed_mode(Plan &p) {
   return SHT_OK;
 }
 
-// Column tiles per workgroup of the streaming inverse: at most 8, and at
-// least 3 workgroups per m once there are more than 3 tiles, the chunks
-// balanced (one workgroup per CU runs, so a short last chunk or too few
-// workgroups leaves CUs idle).  Measured at T170 (split-BF16 x6): 776
-// fields 4 / 8 / 12 / 16 / 32 tiles 225 / 212 / 211 / 219 / 252 us; 200
-// fields (25 tiles) 8 tiles 52.1 us, 6 tiles 44.1 us; 33 fields (5 tiles)
-// 5 tiles 15.6 us, 2 tiles 13.6 us.
+// Column tiles per workgroup of the streaming inverse: 8, up to 16 where
+// that still leaves each m six workgroups, and at least two workgroups per m,
+// the chunks balanced (one workgroup per CU runs, so a short last chunk or too
+// few workgroups leave CUs idle, while each chunk loads its m's table again).
+// Measured at T170 (split-BF16 x6), chunks of at most 6 / 8 / 12 / 16: 776
+// fields 164.9 / 159.7 / 158.2 / 153.9 us, 388 fields 88.6 / 84.4 / 84.1 /
+// 87.7; at least three workgroups per m against two: 33 fields 14.6 / 14.0, 60
+// fields 17.8 / 16.5, 97 fields 25.9 / 25.7.
 int stream_chunk(int nct) {
-  if (nct <= 3) return nct;
-  const int nchunks = std::max(3, (nct + 7) / 8);
+  if (nct <= 2) return nct;
+  const int most = std::min(16, std::max(8, nct / 6)), nchunks = std::max(2, (nct + most - 1) / most);
   return (nct + nchunks - 1) / nchunks;
 }
 
@@ -1215,11 +1236,10 @@ int inv_nsl(const Plan &p, int shape, const double *spec, float *four, int nf, h
   }
   if (shape == SHT_SHAPE_STAGED) {
     if (!mixed_stream_available(p)) return fail(SHT_ERR_UNSUPPORTED, "mixed inverse: streaming shape needs <= 128 latitude pairs");
-    // loads 4 tiles ahead (T170, 776 fields, split-BF16 x6, 8 tiles per
-    // workgroup: 2 / 3 / 4 tiles ahead 219 / 216 / 212 us)
+    // each half of the waves loads two of its tiles (every second one) ahead
     const int cs = stream_chunk(nct);
-    launch_kernel(geo.stream ? leg_inv_mixed_stream_kernel<MODE, NSL, true, 4> : leg_inv_mixed_stream_kernel<MODE, NSL, false, 4>,
-                  xcd_m_blocks(p, 0, (nct + cs - 1) / cs), 512, 0, s, spec, four,
+    launch_kernel(geo.stream ? leg_inv_mixed_stream_kernel<MODE, NSL, true, 2> : leg_inv_mixed_stream_kernel<MODE, NSL, false, 2>,
+                  xcd_m_blocks(p, 0, (nct + cs - 1) / cs), 1024, 0, s, spec, four,
                   static_cast<const uint16_t *>(p.Linv), p.loff_inv, p.lexp_inv, p.xcd_m[0],
                   p.xcd_mlen[0], p.N, p.P2, p.P2p, ncol, nct, cs, geo);
     SHT_HIP(hipGetLastError());
