@@ -201,56 +201,79 @@ __device__ __forceinline__ void slice_mac2(const uint4 (&pa0)[3], const uint4 (&
 // values padded to 40 (80 bytes): eight lanes reading the same K octet of
 // consecutive columns then hit eight different 16-byte bank groups.
 constexpr int kRowPitch = 40;
-// Every wave converts whole groups (wave w of NW takes groups w, w+NW, ...): lane l
-// reads the 8 values K = 8 (l/16) .. +7 of column l % 16 (load(g, k, c) returns
-// the FP64 value or 0 outside the tile), the FP16 exponent comes from the
-// maximum over the group's 32 values (a 4-lane shuffle reduction), and the
-// lane writes each of its pieces as one 16-byte LDS store -- already the
-// matrix-core B layout.  A wave issues the loads of NIT groups before it
-// converts any, so one memory latency covers them (groups past ngroups load
-// group 0 again and are not stored).  Group g lands in LDS slot slot(g), so a
-// caller can stage only the groups that hold data.
-template <int MODE, int NIT, int NW, class Slot, class Load>
-__device__ __forceinline__ void stage_data(uint16_t *bt, int *ebits, int ngroups, Slot slot, Load load,
-                                           int tid) {
+// A lane of the converting wave holds 4 K values (4 k4 .. 4 k4 + 3, k4 =
+// lane / 8) of two neighbouring columns (2 c2, 2 c2 + 1, c2 = lane % 8), so its
+// loads take both columns at once (16 bytes of spectra, 8 of Fourier data;
+// one column and 8 K values per lane took twice as many load instructions:
+// split-BF16 x6, T170, 776 fields, inverse 151 -> 138 us, T85, 388 fields 22.0
+// -> 21.4 and forward 19.4 -> 19.1; scaled FP16 forward 17.0 -> 16.2).
+// Splits the values of group g, v[K value][column], into LDS: the FP16
+// exponent comes from the maximum over the group's 32 values of a column (an
+// 8-lane shuffle reduction), and each piece of a column leaves as one 8-byte
+// store -- already the matrix-core B layout.
+template <int MODE>
+__device__ __forceinline__ void put_group(uint16_t *bt, int *ebits, int g, int lane, const float (&v)[4][2]) {
   constexpr int NP = Form<MODE>::NP;
-  const int lane = tid & 63, c = lane & 15, k8 = lane >> 4;
-  using T = decltype(load(0, 0, 0));  // double (spectra) or float (Fourier data)
+  const int c2 = lane & 7, k4 = lane >> 3;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    int e = 0;
+    if constexpr (Form<MODE>::kScaled) {
+      float mx = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mx = fmax(mx, fabs(v[i][h]));
+#pragma unroll
+      for (int s = 8; s < 64; s <<= 1) mx = fmax(mx, __shfl_xor(mx, s));
+      e = mx > 0 ? 13 - ilogb(mx) : 0;
+      if (k4 == 0) ebits[g * 16 + 2 * c2 + h] = e;
+    }
+    uint32_t w[3][2];
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      uint16_t p0[3], p1[3];
+      split<MODE>(Form<MODE>::kScaled ? ldexp(v[i][h], e) : v[i][h], p0);
+      split<MODE>(Form<MODE>::kScaled ? ldexp(v[i + 1][h], e) : v[i + 1][h], p1);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[q][i >> 1] = p0[q] | ((uint32_t)p1[q] << 16);
+    }
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+      *reinterpret_cast<uint2 *>(bt + (((size_t)g * NP + q) * 16 + 2 * c2 + h) * kRowPitch + k4 * 4) =
+          make_uint2(w[q][0], w[q][1]);
+  }
+}
+// Every wave converts whole groups (wave w of NW takes groups w, w+NW, ...):
+// load(g, k, c) returns columns c, c + 1 (c even) at K index k, values in .x
+// and .y, valid(g, k, c) whether they lie inside the tile (zero otherwise).  A
+// wave issues the loads of NIT groups before it converts any, so one memory
+// latency covers them (groups past ngroups load group 0 again and are not
+// stored).  Group g lands in LDS slot slot(g), so a caller can stage only the
+// groups that hold data.
+template <int MODE, int NIT, int NW, class Slot, class Load, class Valid>
+__device__ __forceinline__ void stage_data(uint16_t *bt, int *ebits, int ngroups, Slot slot, Load load, Valid valid,
+                                           int tid) {
+  const int lane = tid & 63, c = 2 * (lane & 7), k4 = lane >> 3;
+  using T2 = decltype(load(0, 0, 0));  // double2 (spectra) or float2 (Fourier data)
   for (int g0 = __builtin_amdgcn_readfirstlane(tid >> 6); g0 < ngroups; g0 += NW * NIT) {
-    T v[NIT][8];
+    T2 v[NIT][4];
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       const int g = g0 + NW * it < ngroups ? g0 + NW * it : 0;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[it][i] = load(g, k8 * 8 + i, c);
+      for (int i = 0; i < 4; ++i) v[it][i] = load(g, k4 * 4 + i, c);
     }
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
       if (g0 + NW * it >= ngroups) break;
-      const int g = slot(g0 + NW * it);
-      int e = 0;
-      if constexpr (Form<MODE>::kScaled) {
-        T mx = 0;
+      float f[4][2];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) mx = fmax(mx, fabs(v[it][i]));
-        mx = fmax(mx, __shfl_xor(mx, 16));
-        mx = fmax(mx, __shfl_xor(mx, 32));
-        e = mx > 0 ? 13 - ilogb(mx) : 0;
-        if (k8 == 0) ebits[g * 16 + c] = e;
+      for (int i = 0; i < 4; ++i) {
+        // split as FP32: see split(float)
+        const bool ok = valid(g0 + NW * it, k4 * 4 + i, c);
+        f[i][0] = ok ? (float)v[it][i].x : 0.0f;
+        f[i][1] = ok ? (float)v[it][i].y : 0.0f;
       }
-      uint32_t w[3][4];
-#pragma unroll
-      for (int i = 0; i < 8; i += 2) {
-        uint16_t p0[3], p1[3];
-        split<MODE>(Form<MODE>::kScaled ? ldexp(v[it][i], e) : v[it][i], p0);
-        split<MODE>(Form<MODE>::kScaled ? ldexp(v[it][i + 1], e) : v[it][i + 1], p1);
-#pragma unroll
-        for (int q = 0; q < 3; ++q) w[q][i >> 1] = p0[q] | ((uint32_t)p1[q] << 16);
-      }
-#pragma unroll
-      for (int q = 0; q < NP; ++q)
-        *reinterpret_cast<uint4 *>(bt + (((size_t)g * NP + q) * 16 + c) * kRowPitch + k8 * 8) =
-            make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
+      put_group<MODE>(bt, ebits, slot(g0 + NW * it), lane, f);
     }
   }
 }
@@ -433,13 +456,23 @@ __device__ __forceinline__ void leg_inv_mixed_item(
     const int j = g / ng, r = g - j * ng, par = r >= nsl;
     return j * NG + par * NSL + r - par * nsl;
   };
-  stage_data<MODE, stage_iters<CT * NG, NW>(), NW>(bt, ebits, nc * ng, slot, [&](int g, int k, int c) {
+  struct At {
+    int par, kk, cc;
+  };
+  auto at = [&](int g, int k, int c) {
     const int j = g / ng, r = g - j * ng, par = r >= nsl, s = r - par * nsl;
-    const int kk = s * 32 + k, cc = j * 16 + c;
-    const bool v = kk < (par ? ko : ke) && ct0 * 16 + cc < ncol;
-    const double x = sm[(size_t)(v ? 2 * kk + par : 0) * ncol + (v ? cc : 0)];
-    return v ? (float)x : 0.0f;  // split as FP32: see split(float)
-  }, tid);
+    return At{par, s * 32 + k, j * 16 + c};
+  };
+  auto valid = [&](int g, int k, int c) {
+    const At a = at(g, k, c);
+    return a.kk < (a.par ? ko : ke) && ct0 * 16 + a.cc < ncol;
+  };
+  stage_data<MODE, stage_iters<CT * NG, NW>(), NW>(bt, ebits, nc * ng, slot, [&](int g, int k, int c) {
+    const At a = at(g, k, c);
+    // the caller's spectra may be only 8-byte aligned: two loads (merged)
+    const double *x = sm + (valid(g, k, c) ? (size_t)(2 * a.kk + a.par) * ncol + a.cc : 0);
+    return make_double2(x[0], x[1]);
+  }, valid, tid);
   __syncthreads();
   for (int rt = wave; rt < rtiles; rt += NW) {
     if (rt != wave) load_a(rt);
@@ -705,12 +738,22 @@ __device__ __forceinline__ void leg_fwd_mixed_item(
 #pragma unroll
       for (int q = 0; q < 3; ++q) pa[s][q] = (q < NP) ? a_frag(wave, s, q) : make_uint4(0, 0, 0, 0);
   }
+  struct At {
+    int par, p, cc;
+  };
+  auto at = [&](int g, int k, int c) {
+    const int j = g / NG, par = (g % NG) / NSL, s = g % NSL;
+    return At{par, s * 32 + k, ct0 * 16 + j * 16 + c};
+  };
+  auto valid = [&](int g, int k, int c) {
+    const At a = at(g, k, c);
+    return a.p < P2 && a.cc < ncol;
+  };
   stage_data<MODE, stage_iters<CT * NG, NW>(), NW>(bt, ebits, nc * NG, [](int g) { return g; }, [&](int g, int k, int c) {
-    const int j = g / NG, par = (g % NG) / NSL, s = g % NSL, p = s * 32 + k, cc = ct0 * 16 + j * 16 + c;
-    const bool v = p < P2 && cc < ncol;
-    const float x = four[geo.at(v ? p : 0, m, par, v ? cc : ct0 * 16)];
-    return v ? x : 0.0f;
-  }, tid);
+    const At a = at(g, k, c);
+    const bool v = valid(g, k, c);
+    return *reinterpret_cast<const float2 *>(four + geo.at(v ? a.p : 0, m, a.par, v ? a.cc : ct0 * 16));
+  }, valid, tid);
   __syncthreads();
   for (int u = wave; u < nunits; u += NW) {
     const int par = u / nrt, rt = u % nrt;
@@ -978,34 +1021,27 @@ __global__ __launch_bounds__(1024) void leg_inv_mixed_stream_kernel(
   // slice gs, LDS slot gpar NSL + gs
   const bool stg = w8 < 2 * nsl;
   const int gpar = w8 >= nsl, gs = w8 - gpar * nsl, kend = gpar ? ko : ke;
-  auto load = [&](int j, double (&v)[8]) {
-    const int col = (j0 + j) * 16 + c;
+  const int lc = 2 * (lane & 7), lk = (lane >> 3) * 4;  // see put_group
+  auto load = [&](int j, double2 (&v)[4]) {
+    const int col = (j0 + j) * 16 + lc;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int kk = gs * 32 + k8 * 8 + i;
-      const bool ok = kk < kend && col < ncol;
-      v[i] = sm[(size_t)(ok ? 2 * kk + gpar : 0) * ncol + (ok ? col : 0)];
+    for (int i = 0; i < 4; ++i) {
+      const int kk = gs * 32 + lk + i;
+      const double *x = sm + (kk < kend && col < ncol ? (size_t)(2 * kk + gpar) * ncol + col : 0);
+      v[i] = make_double2(x[0], x[1]);
     }
   };
-  auto put = [&](int j, const double (&v)[8]) {
+  auto put = [&](int j, const double2 (&v)[4]) {
     unsigned char *b = lds + half * kBuf;  // j & 1 == half
-    const int col = (j0 + j) * 16 + c;
-    float f[8];
+    const int col = (j0 + j) * 16 + lc;
+    float f[4][2];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int kk = gs * 32 + k8 * 8 + i;
-      f[i] = kk < kend && col < ncol ? (float)v[i] : 0.0f;  // split as FP32: see split(float)
+    for (int i = 0; i < 4; ++i) {
+      const bool ok = gs * 32 + lk + i < kend && col < ncol;
+      f[i][0] = ok ? (float)v[i].x : 0.0f;  // split as FP32: see split(float)
+      f[i][1] = ok ? (float)v[i].y : 0.0f;
     }
-    const int e = col_exponent<MODE>(f);
-    uint4 pc[3];
-    split8<MODE>(f, e, pc);
-    const int g = gpar * NSL + gs;
-    if constexpr (Form<MODE>::kScaled)
-      if (k8 == 0) reinterpret_cast<int *>(b + One::bt)[g * 16 + c] = e;
-    uint16_t *bt = reinterpret_cast<uint16_t *>(b);
-#pragma unroll
-    for (int q = 0; q < NP; ++q)
-      *reinterpret_cast<uint4 *>(bt + ((size_t)(g * NP + q) * 16 + c) * kRowPitch + k8 * 8) = pc[q];
+    put_group<MODE>(reinterpret_cast<uint16_t *>(b), reinterpret_cast<int *>(b + One::bt), gpar * NSL + gs, lane, f);
   };
   const double ea = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m + half]) : 1.0;
   float *ob = reinterpret_cast<float *>(lds + 2 * kBuf) + wave * (16 * kPitch);
@@ -1033,7 +1069,7 @@ __global__ __launch_bounds__(1024) void leg_inv_mixed_stream_kernel(
   };
   // column tile j: the staging half converts its loaded values into buffer j
   // % 2, then (barrier) loads its tile after the next PD - 1, and all multiply
-  double v[PD][8];
+  double2 v[PD][4];
   if (stg) {
 #pragma unroll
     for (int d = 0; d < PD; ++d)
