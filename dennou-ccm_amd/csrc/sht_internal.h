@@ -147,6 +147,16 @@ struct FourGeom {
   __host__ __device__ size_t at(int p, int m, int par, int c) const {
     return ((((size_t)(c >> lg) * P2 + p) * M1 + m) * 2 + par) * ((size_t)1 << lg) + (c & ((1 << lg) - 1));
   }
+  // The same split for a 16-column tile from column c0 (a multiple of 16, so
+  // inside one group): at(p, m, par, c0 + c) = tile(m, c0) + p pair() + par
+  // parity() + c.  tile() is the same in all lanes and the rest below 2^22
+  // (M1 2 cgs <= 8192, 512 latitudes), so an access is a scalar base and one
+  // 32-bit lane offset.
+  __device__ size_t tile(int m, int c0) const {
+    return ((((size_t)(c0 >> lg) * P2) * M1 + m) * 2 << lg) + (c0 & ((1 << lg) - 1));
+  }
+  __device__ unsigned pair() const { return (unsigned)M1 * 2u << lg; }
+  __device__ unsigned parity() const { return 1u << lg; }
 };
 // Store of the Fourier intermediate; NT (non-temporal) is a template
 // argument of the writing kernels because a run-time choice between the two

@@ -311,11 +311,6 @@ constexpr int kOutPitch = 36;
 // once, and the table fragments fetched per column.  Results leave through a
 // per-wave LDS transpose as 16-byte stores of 4 consecutive columns (the
 // Fourier layout keeps a field group's 2G columns contiguous).
-// One column tile per workgroup with at most two K slices (N <= 127) asks
-// the compiler for 5 waves per SIMD, so a T85 batch of 97 fields (1144
-// workgroups) is resident at once (measured at T85: neutral at 97 fields, 6 %
-// faster at 388; the six-product form spills two registers for it).  With
-// more slices the hint would spill heavily.
 // Store of the FP32 Fourier intermediate: COH = device-coherent (agent-scope
 // relaxed atomic stores, 8 bytes each), for data another workgroup of the
 // same kernel reads; otherwise put_four.
@@ -331,15 +326,6 @@ __device__ __forceinline__ void put_four4(float *dst, f4 v) {
     put_four<NT>(reinterpret_cast<f4 *>(dst), v);
   }
 }
-template <bool NT, bool COH>
-__device__ __forceinline__ void put_four1(float *dst, float v) {
-  if constexpr (COH)
-    __hip_atomic_store(reinterpret_cast<unsigned *>(dst), __float_as_uint(v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  else
-    put_four<NT>(dst, v);
-}
-
 // One row tile rt (16 latitude pairs, its table fragments pa) against one
 // staged column tile jt (groups par * NSL + s at bt, FP16 exponents at
 // ebits): the nsl K slices' products summed in FP64 per parity, then the FP32
@@ -350,7 +336,7 @@ __device__ __forceinline__ void inv_tile(const uint16_t *bt, const int *ebits, f
                                          const uint4 (&pa)[2][NSL][3], double ea0, double ea1, int nsl,
                                          float *__restrict__ four, FourGeom geo, int P2, int ncol, int m,
                                          int rt, int jt, int lane) {
-  const int r16 = lane & 15, kq = lane >> 4, col = jt * 16 + r16;
+  const int r16 = lane & 15, kq = lane >> 4;
   d4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
 #pragma unroll
   for (int s = 0; s < NSL; ++s) {
@@ -362,33 +348,20 @@ __device__ __forceinline__ void inv_tile(const uint16_t *bt, const int *ebits, f
     const double sc1 = Form<MODE>::kScaled ? ea1 * ldexp(1.0, -ebits[(NSL + s) * 16 + r16]) : 1.0;
     slice_mac2<MODE>(pa[0][s], pb0, sc0, acc[0], pa[1][s], pb1, sc1, acc[1]);
   }
-  if (geo.lg >= 2) {
-    // 4 consecutive columns per lane: through the wave's LDS patch
-    // [16 pairs][2 parities][16 columns] (row pitch kOutPitch); the
-    // padding columns of the last field group are written too (zeros)
+  // 4 consecutive columns per lane: through the wave's LDS patch
+  // [16 pairs][2 parities][16 columns] (row pitch kOutPitch); the padding
+  // columns of the last field group are written too (zeros)
 #pragma unroll
-    for (int par = 0; par < 2; ++par)
+  for (int par = 0; par < 2; ++par)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ob[(kq * 4 + i) * kOutPitch + par * 16 + r16] = (float)acc[par][i];
-    const int cend = geo.nfg << geo.lg;
+    for (int i = 0; i < 4; ++i) ob[(kq * 4 + i) * kOutPitch + par * 16 + r16] = (float)acc[par][i];
+  float *out = four + geo.tile(m, jt * 16);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int q = lane + 64 * h, pl = q >> 3, par = (q >> 2) & 1, c4 = (q & 3) * 4;
-      const int p = rt * 16 + pl, cc = jt * 16 + c4;
-      const f4 v = *reinterpret_cast<const f4 *>(ob + pl * kOutPitch + par * 16 + c4);
-      if (p < P2 && cc < cend) put_four4<NT, COH>(four + geo.at(p, m, par, cc), v);
-    }
-  } else if (col < ncol) {
-    // field groups of fewer than 4 columns: none since groups hold at least
-    // 8 fields (layout_group), but without this path the compiler spills 94
-    // registers of the T85 six-product inverse (2 with it)
-#pragma unroll
-    for (int par = 0; par < 2; ++par)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int p = rt * 16 + kq * 4 + i;
-        if (p < P2) put_four1<NT, COH>(four + geo.at(p, m, par, col), (float)acc[par][i]);
-      }
+  for (int h = 0; h < 2; ++h) {
+    const int q = lane + 64 * h, pl = q >> 3, par = (q >> 2) & 1, c4 = (q & 3) * 4;
+    const int p = rt * 16 + pl;
+    const f4 v = *reinterpret_cast<const f4 *>(ob + pl * kOutPitch + par * 16 + c4);
+    if (p < P2) put_four4<NT, COH>(out + (p * geo.pair() + par * geo.parity() + c4), v);
   }
 }
 
@@ -414,8 +387,10 @@ struct InvItemLds {
 // per-wave LDS transpose as 16-byte stores of 4 consecutive columns (the
 // Fourier layout keeps a field group's 2G columns contiguous).  This is the
 // work of one (m, column tile t) item, with its LDS at lds; COH stores the
-// intermediate device-coherently (the fused kernel).
-template <int MODE, int NSL, int CT, bool NT, int NW, bool COH>
+// intermediate device-coherently (the fused kernel); ONE: at most NW row tiles,
+// one per wave (without the loop that loads the next row tile's fragments the
+// T85 six-product form takes 78 registers instead of spilling 74 of 96).
+template <int MODE, int NSL, int CT, bool NT, int NW, bool COH, bool ONE>
 __device__ __forceinline__ void leg_inv_mixed_item(
     unsigned char *lds, const double *__restrict__ spec, float *__restrict__ four,
     const uint16_t *__restrict__ L, const int *__restrict__ loff, const int *__restrict__ lexp, int N,
@@ -475,7 +450,8 @@ __device__ __forceinline__ void leg_inv_mixed_item(
   }, valid, tid);
   __syncthreads();
   for (int rt = wave; rt < rtiles; rt += NW) {
-    if (rt != wave) load_a(rt);
+    if constexpr (!ONE)
+      if (rt != wave) load_a(rt);
     const double ea0 = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m]) : 1.0;
     const double ea1 = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m + 1]) : 1.0;
 #pragma unroll
@@ -485,16 +461,18 @@ __device__ __forceinline__ void leg_inv_mixed_item(
                                    obuf + wave * (16 * kOutPitch), pa, ea0, ea1, nsl, four, geo, P2, ncol,
                                    m, rt, ct0 + j, lane);
     }
+    if constexpr (ONE) break;
   }
 }
 
 // One column tile per workgroup with at most two K slices (N <= 127) asks
 // the compiler for 5 waves per SIMD, so a T85 batch of 97 fields (1144
 // workgroups) is resident at once (measured at T85: neutral at 97 fields, 6 %
-// faster at 388; the six-product form spills two registers for it).  With
-// more slices the hint would spill heavily.
-template <int MODE, int NSL, int CT, bool NT, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu((CT == 1 && NSL <= 2) ? 5 : 1))) void
+// faster at 388); four in the six-product form with several row tiles a wave,
+// which spills at five.  With more slices the hint would spill heavily.
+template <int MODE, int NSL, int CT, bool NT, int NW, bool ONE>
+__global__ __launch_bounds__(NW * 64) __attribute__((
+    amdgpu_waves_per_eu((CT == 1 && NSL <= 2) ? (!ONE && Form<MODE>::NP == 3 ? 4 : 5) : 1))) void
 leg_inv_mixed_kernel(
     const double *__restrict__ spec, float *__restrict__ four, const uint16_t *__restrict__ L,
     const int *__restrict__ loff, const int *__restrict__ lexp, const int *__restrict__ mlist,
@@ -502,7 +480,7 @@ leg_inv_mixed_kernel(
   __shared__ __align__(16) unsigned char lds[InvItemLds<MODE, NSL, CT, NW>::bytes];
   int m, t;
   if (!xcd_m_block(blockIdx.x, mlist, mlen, (nct + CT - 1) / CT, m, t)) return;
-  leg_inv_mixed_item<MODE, NSL, CT, NT, NW, false>(lds, spec, four, L, loff, lexp, N, P2, P2p, ncol, nct,
+  leg_inv_mixed_item<MODE, NSL, CT, NT, NW, false, ONE>(lds, spec, four, L, loff, lexp, N, P2, P2p, ncol, nct,
                                                    geo, m, t, threadIdx.x);
 }
 
@@ -667,7 +645,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void i
     if (item >= 0) {
       const int y = item >> 24, i = item & 0xffffff;
       const int t = i / a.mlen, m = a.mlist[y * a.mlen + i % a.mlen];
-      leg_inv_mixed_item<MODE, NSL, 1, false, 4, true>(lds, a.spec, a.four, a.L, a.loff, a.lexp, a.N, a.P2,
+      leg_inv_mixed_item<MODE, NSL, 1, false, 4, true, false>(lds, a.spec, a.four, a.L, a.loff, a.lexp, a.N, a.P2,
                                                        a.P2p, a.ncol, a.nct, a.geo, m, t, ltid);
       // this thread's coherent stores have completed; after the barrier
       // every thread's have, and the column tile counts one more m
@@ -738,21 +716,15 @@ __device__ __forceinline__ void leg_fwd_mixed_item(
 #pragma unroll
       for (int q = 0; q < 3; ++q) pa[s][q] = (q < NP) ? a_frag(wave, s, q) : make_uint4(0, 0, 0, 0);
   }
-  struct At {
-    int par, p, cc;
-  };
-  auto at = [&](int g, int k, int c) {
-    const int j = g / NG, par = (g % NG) / NSL, s = g % NSL;
-    return At{par, s * 32 + k, ct0 * 16 + j * 16 + c};
-  };
+  // columns past ncol lie in the last group's padding: loaded, not used
+  const unsigned pp = geo.pair();
   auto valid = [&](int g, int k, int c) {
-    const At a = at(g, k, c);
-    return a.p < P2 && a.cc < ncol;
+    return (g % NSL) * 32 + k < P2 && (ct0 + g / NG) * 16 + c < ncol;
   };
   stage_data<MODE, stage_iters<CT * NG, NW>(), NW>(bt, ebits, nc * NG, [](int g) { return g; }, [&](int g, int k, int c) {
-    const At a = at(g, k, c);
-    const bool v = valid(g, k, c);
-    return *reinterpret_cast<const float2 *>(four + geo.at(v ? a.p : 0, m, a.par, v ? a.cc : ct0 * 16));
+    const int par = (g % NG) / NSL, p = (g % NSL) * 32 + k;
+    const float *base = four + geo.tile(m, (ct0 + g / NG) * 16) + par * geo.parity();
+    return *reinterpret_cast<const float2 *>(base + ((p < P2 ? p : 0) * pp + c));
   }, valid, tid);
   __syncthreads();
   for (int u = wave; u < nunits; u += NW) {
@@ -823,10 +795,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void l
   int m, t;
   if (!xcd_m_block(blockIdx.x - g.blk0, g.mlist, g.mlen, g.nct, m, t)) return;
   if (g.nsl == 1)
-    leg_inv_mixed_item<MODE, 1, 1, NT, 4, false>(lds, g.spec_in, g.four, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol,
+    leg_inv_mixed_item<MODE, 1, 1, NT, 4, false, true>(lds, g.spec_in, g.four, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol,
                                                  g.nct, g.geo, m, t, threadIdx.x);
   else
-    leg_inv_mixed_item<MODE, 2, 1, NT, 4, false>(lds, g.spec_in, g.four, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol,
+    leg_inv_mixed_item<MODE, 2, 1, NT, 4, false, true>(lds, g.spec_in, g.four, g.L, g.loff, g.lexp, g.N, g.P2, g.P2p, g.ncol,
                                                  g.nct, g.geo, m, t, threadIdx.x);
 }
 
@@ -1045,7 +1017,6 @@ __global__ __launch_bounds__(1024) void leg_inv_mixed_stream_kernel(
   };
   const double ea = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m + half]) : 1.0;
   float *ob = reinterpret_cast<float *>(lds + 2 * kBuf) + wave * (16 * kPitch);
-  const int cend = geo.nfg << geo.lg;
   auto multiply = [&](int j) {
     const unsigned char *b = lds + (j & 1) * kBuf;
     const uint16_t *bt = reinterpret_cast<const uint16_t *>(b);
@@ -1063,13 +1034,120 @@ __global__ __launch_bounds__(1024) void leg_inv_mixed_stream_kernel(
     // columns]; the padding columns of the last field group are written too
 #pragma unroll
     for (int i = 0; i < 4; ++i) ob[(k8 * 4 + i) * kPitch + c] = (float)acc[i];
-    const int pl = lane >> 2, c4 = (lane & 3) * 4, p = w8 * 16 + pl, cc = (j0 + j) * 16 + c4;
+    const int pl = lane >> 2, c4 = (lane & 3) * 4, p = w8 * 16 + pl;
     const f4 v = *reinterpret_cast<const f4 *>(ob + pl * kPitch + c4);
-    if (p < P2 && cc < cend) put_four<NT>(reinterpret_cast<f4 *>(four + geo.at(p, m, half, cc)), v);
+    if (p < P2)
+      put_four<NT>(reinterpret_cast<f4 *>(four + geo.tile(m, (j0 + j) * 16) + (p * geo.pair() + half * geo.parity() + c4)),
+                   v);
   };
   // column tile j: the staging half converts its loaded values into buffer j
   // % 2, then (barrier) loads its tile after the next PD - 1, and all multiply
   double2 v[PD][4];
+  if (stg) {
+#pragma unroll
+    for (int d = 0; d < PD; ++d)
+      if (2 * d + half < nj) load(2 * d + half, v[d]);
+  }
+  for (int j = 0; j < nj; j += 2 * PD) {
+#pragma unroll
+    for (int d = 0; d < 2 * PD; ++d) {
+      if (j + d >= nj) break;
+      const bool mine = stg && (d & 1) == half;
+      if (mine) put(j + d, v[d / 2]);
+      __syncthreads();
+      if (mine && j + d + 2 * PD < nj) load(j + d + 2 * PD, v[d / 2]);
+      if (mma) multiply(j + d);
+    }
+  }
+}
+
+// Streaming forward (shape TILE on grids of 128 latitude pairs): the inverse's
+// scheme with the roles of degrees and pairs exchanged.  Workgroup = (m, a
+// chunk of cs column tiles) of sixteen waves; wave w holds the table of unit w
+// (parity w / nrt, 16-degree row tile w % nrt; at most 16 units) for the whole
+// chunk while the Fourier tiles pass through two LDS buffers, staged by the
+// two halves of the waves in turn (wave w: group w % 8 of 2 NSL <= 8).  Per
+// output tile the products and sums of leg_fwd_mixed_item in its order.  One
+// workgroup per CU, so its registers (128 per lane) decide: PD = 1 in the
+// forms whose table and staging would spill with 2 (x6, 776 fields: 216 us
+// with 15 values spilled, 137 us without).  Times: fwd_streams.
+template <int MODE, int NSL, int PD>
+__global__ __launch_bounds__(1024) void leg_fwd_mixed_stream_kernel(
+    const float *__restrict__ four, double *__restrict__ spec, const uint16_t *__restrict__ L,
+    const int *__restrict__ loff, const int *__restrict__ lexp, const int *__restrict__ mlist,
+    int mlen, int N, int P2, int P2p32, int ncol, int nct, int cs, FourGeom geo) {
+  constexpr int NP = Form<MODE>::NP;
+  using One = FwdItemLds<MODE, NSL, 1>;
+  __shared__ __align__(16) unsigned char lds[2 * One::bytes];
+  int m, t;
+  if (!xcd_m_block(blockIdx.x, mlist, mlen, (nct + cs - 1) / cs, m, t)) return;
+  const int wave = wave_id(), w8 = wave & 7, half = wave >> 3;
+  const int lane = threadIdx.x & 63, c = lane & 15, k8 = lane >> 4;
+  const int j0 = t * cs, nj = nct - j0 < cs ? nct - j0 : cs;
+  const int nn = N - m + 1, ke = (nn + 1) >> 1;
+  const int KR = (ke + 15) & ~15, nrt = KR >> 4;
+  const uint16_t *__restrict__ Lm = L + loff[m];
+  // this wave's unit
+  const bool mma = wave < 2 * nrt;
+  const int par = wave >= nrt, rt = wave - par * nrt, kc = par ? (nn >> 1) : ke;
+  uint4 pa[NSL][3];
+  if (mma) {
+#pragma unroll
+    for (int s = 0; s < NSL; ++s)
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        pa[s][q] = q < NP ? *reinterpret_cast<const uint4 *>(
+                                Lm + ((size_t)(par * NP + q) * KR + rt * 16 + c) * P2p32 + s * 32 + k8 * 8)
+                          : make_uint4(0, 0, 0, 0);
+  }
+  // this wave's staging: tiles j with j % 2 = half, group w8: parity, K slice
+  const bool stg = w8 < 2 * NSL;
+  const int gpar = w8 >= NSL, gs = w8 - gpar * NSL;
+  const int lc = 2 * (lane & 7), lp = gs * 32 + (lane >> 3) * 4;  // see put_group
+  const unsigned pp = geo.pair();
+  auto load = [&](int j, float2 (&v)[4]) {
+    // columns past ncol lie in the last group's padding: loaded, not used
+    const float *base = four + geo.tile(m, (j0 + j) * 16) + gpar * geo.parity();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const float2 *>(base + ((lp + i < P2 ? lp + i : 0) * pp + lc));
+  };
+  auto put = [&](int j, const float2 (&v)[4]) {
+    unsigned char *b = lds + half * One::bytes;  // j & 1 == half
+    const int col = (j0 + j) * 16 + lc;
+    float f[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool ok = lp + i < P2 && col < ncol;
+      f[i][0] = ok ? v[i].x : 0.0f;
+      f[i][1] = ok ? v[i].y : 0.0f;
+    }
+    put_group<MODE>(reinterpret_cast<uint16_t *>(b), reinterpret_cast<int *>(b + One::bt), w8, lane, f);
+  };
+  const double ea = Form<MODE>::kScaled ? ldexp(1.0, -lexp[2 * m + par]) : 1.0;
+  double *__restrict__ sm = spec + (size_t)coef_off(N, m) * ncol;
+  const int k0 = rt * 16 + k8 * 4;                            // the lane's first degree row
+  const unsigned out0 = (unsigned)(2 * k0 + par) * ncol + c;  // below 2^32: 256 rows of 2 kmax
+  auto multiply = [&](int j) {
+    const unsigned char *b = lds + (j & 1) * One::bytes;
+    const uint16_t *bt = reinterpret_cast<const uint16_t *>(b);
+    const int *ebits = reinterpret_cast<const int *>(b + One::bt);
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < NSL; ++s) {
+      const int g = par * NSL + s;
+      uint4 pb[3];
+      load_pb<MODE>(bt, g, k8, c, pb);
+      slice_mac<MODE>(pa[s], pb, Form<MODE>::kScaled ? ea * ldexp(1.0, -ebits[g * 16 + c]) : 1.0, acc);
+    }
+    if ((j0 + j) * 16 + c < ncol) {
+      // the tile's column is the same in all lanes: a scalar base, one lane offset
+      double *__restrict__ st = sm + (size_t)(j0 + j) * 16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (k0 + i < kc) put_spec(st + (size_t)(2 * i) * ncol + out0, acc[i]);
+    }
+  };
+  float2 v[PD][4];
   if (stg) {
 #pragma unroll
     for (int d = 0; d < PD; ++d)
@@ -1284,9 +1362,13 @@ int inv_nsl(const Plan &p, int shape, const double *spec, float *four, int nf, h
   // KSPLIT: one column tile per workgroup; TILE: two.  Four waves (eight,
   // as the forward takes them at T170, measured slower here: 242 against
   // 217 us for TILE at T170, 776 fields).
-  auto kern = shape == SHT_SHAPE_TILE
-                  ? (geo.stream ? leg_inv_mixed_kernel<MODE, NSL, 2, true, 4> : leg_inv_mixed_kernel<MODE, NSL, 2, false, 4>)
-                  : (geo.stream ? leg_inv_mixed_kernel<MODE, NSL, 1, true, 4> : leg_inv_mixed_kernel<MODE, NSL, 1, false, 4>);
+  auto pick = [&](auto one) {
+    constexpr bool ONE = decltype(one)::value;
+    return shape == SHT_SHAPE_TILE
+               ? (geo.stream ? leg_inv_mixed_kernel<MODE, NSL, 2, true, 4, ONE> : leg_inv_mixed_kernel<MODE, NSL, 2, false, 4, ONE>)
+               : (geo.stream ? leg_inv_mixed_kernel<MODE, NSL, 1, true, 4, ONE> : leg_inv_mixed_kernel<MODE, NSL, 1, false, 4, ONE>);
+  };
+  auto kern = p.P2p <= 4 * 16 ? pick(std::true_type{}) : pick(std::false_type{});
   const int ct = shape == SHT_SHAPE_TILE ? 2 : 1;
   launch_kernel(kern, xcd_m_blocks(p, 0, (nct + ct - 1) / ct), 256, 0, s, spec, four,
                 static_cast<const uint16_t *>(p.Linv), p.loff_inv, p.lexp_inv, p.xcd_m[0],
@@ -1361,6 +1443,19 @@ int build_fused(Plan &p) {
   });
 }
 
+// Whether TILE runs as the streaming forward (128 latitude pairs): not between
+// a few column tiles, where the two-tile workgroups fill the chip better, and
+// enough for several workgroups per m.  T170, two-tile workgroups / streaming,
+// us: x6 8 fields 8.4 / 7.1, 33 fields 12.8 / 13.5, 48 fields 13.0 / 13.9, 60
+// fields 16.4 / 16.0, 145 fields 38.2 / 34.9, 388 fields 81.8 / 65.3, 776 fields
+// 161 / 139; BF16 x3 8 fields 6.4 / 5.9, 33 fields 10.2 / 10.8, 388 fields 69.0 /
+// 55.4, 776 fields 129 / 115; scaled FP16 145 fields 32.7 / 32.8, 388 fields
+// 69.8 / 61.6.
+template <int MODE>
+bool fwd_streams(int nf) {
+  return nf <= 24 || nf >= (MODE == SHT_PREC_SPLIT_BF16X6 ? 56 : 192);
+}
+
 template <int MODE, int NSL>
 int fwd_nsl(const Plan &p, int shape, const float *four, double *spec, int nf, hipStream_t s) {
   const int ncol = 2 * nf, nct = (ncol + 15) / 16;
@@ -1371,6 +1466,16 @@ int fwd_nsl(const Plan &p, int shape, const float *four, double *spec, int nf, h
                   four_geom(p, nf));
     SHT_HIP(hipGetLastError());
     return SHT_OK;
+  }
+  if constexpr (NSL <= 4) {
+    if (shape == SHT_SHAPE_TILE && p.P2p == 128 && fwd_streams<MODE>(nf)) {
+      const int cs = stream_chunk(nct);
+      launch_kernel(leg_fwd_mixed_stream_kernel<MODE, NSL, MODE == SHT_PREC_SPLIT_BF16 ? 2 : 1>, xcd_m_blocks(p, 1, (nct + cs - 1) / cs), 1024, 0, s, four,
+                    spec, static_cast<const uint16_t *>(p.Lfwd), p.loff_fwd, p.lexp_fwd, p.xcd_m[1], p.xcd_mlen[1],
+                    p.N, p.P2, roundup(p.P2p, 32), ncol, nct, cs, four_geom(p, nf));
+      SHT_HIP(hipGetLastError());
+      return SHT_OK;
+    }
   }
   // Eight waves share the data tile from 128 latitude pairs (T170: TILE 171
   // against 195 us at 776 fields, 26 against 31 us at 97; KSPLIT neutral),

@@ -348,3 +348,19 @@ def test_fft_block_size_does_not_change_results(prec, N, im, jm, small, big):
     tol = TOL if prec == shtamd.PREC_FP64 else 1e-6
     assert rel(g_small, ref.spec_to_grid(spec[:, :small])) < tol
     p.close()
+
+
+@pytest.mark.parametrize("prec", [shtamd.PREC_SPLIT_BF16, shtamd.PREC_SCALED_FP16, shtamd.PREC_SPLIT_BF16X6])
+@pytest.mark.parametrize("N,im,jm,nf", [(170, 512, 256, 24), (170, 512, 256, 205), (120, 512, 226, 60), (225, 512, 254, 61), (10, 512, 256, 200)])
+def test_mixed_streaming_shapes_bitwise(prec, N, im, jm, nf):
+    """The streaming kernels of the 128-pair grids over one to sixteen table waves,
+    part-filled pair rows, one to several chunks and a part-filled last tile:
+    bitwise the K-split shape's results, either direction."""
+    spec = synth.spectra(N, nf, cfg=9)
+    p = shtamd.Plan(N, im, jm, nf, precision=prec)
+    grid = np.random.default_rng(N).standard_normal((nf, jm, im))
+    p.set_shapes(nf, shtamd.SHAPE_KSPLIT, shtamd.SHAPE_KSPLIT)
+    g0, s0 = run_inverse(p, spec, nf)[0], run_forward(p, grid, nf)
+    p.set_shapes(nf, shtamd.SHAPE_STAGED, shtamd.SHAPE_TILE)
+    assert np.array_equal(run_inverse(p, spec, nf)[0], g0) and np.array_equal(run_forward(p, grid, nf), s0)
+    p.close()
