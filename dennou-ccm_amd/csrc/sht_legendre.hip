@@ -262,8 +262,9 @@ __global__ __launch_bounds__(256) void leg_inv_f64_wave_kernel(
     for (int i = 0; i < 4; ++i) {
       const int p = rt * 16 + i * 4 + kq;
       if (p < P2) {
-        put_four<NT>(out + geo.at(p, m, se, col), acc0[i]);
-        put_four<NT>(out + geo.at(p, m, so, col), acc1[i]);
+        double *o = out + geo.tile(m, ct * 16) + (p * geo.pair() + r16);
+        put_four<NT>(o + se * geo.parity(), acc0[i]);
+        put_four<NT>(o + so * geo.parity(), acc1[i]);
       }
     }
   }
@@ -674,33 +675,32 @@ int fwd_wave_launch(const Plan &p, const double *four, double *spec, int nf, hip
 // until its last unit with a chunk's LDS data read ahead (T170 forward 320
 // against 296 us).
 //
-// Copies rows of 16 columns with NT threads: element e of the block is the
-// column pair c2 = e % 8 of row r = (e / 8) % nrow of column tile
-// j = e / (8 nrow) < CT; src(j, r, col) returns columns col, col + 1 (col even)
-// of the row, zeros outside the data.  Loads are issued NQ at a time before
-// their LDS stores.
+// Copies rows of 16 columns of CT column tiles with NT threads: element e of a
+// tile's block is the column pair c2 = e % 8 of row r = e / 8; src(j, r, col)
+// returns columns col, col + 1 (col even) of the row in tile j (a constant, so
+// tile bases stay scalar), zeros outside the data.  NQ loads per tile are
+// issued before their LDS stores.
 template <int NQ, int NT, int CT, class Src>
 __device__ __forceinline__ void stage_rows(double *sb, int nrow, Src src) {
-  const int nel = CT * nrow * 8;
+  const int nel = nrow * 8;
   for (int e0 = threadIdx.x; e0 < nel; e0 += NQ * NT) {
-    double2 v[NQ];
+    double2 v[CT][NQ];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int e = e0 + q * NT;
-      int r = e >> 3, j = 0;
+    for (int j = 0; j < CT; ++j)
 #pragma unroll
-      for (int i = 1; i < CT; ++i)
-        if (r >= nrow) r -= nrow, ++j;
-      v[q] = e < nel ? src(j, r, 2 * (e & 7)) : make_double2(0.0, 0.0);
-    }
+      for (int q = 0; q < NQ; ++q) {
+        const int e = e0 + q * NT;
+        v[j][q] = e < nel ? src(j, e >> 3, 2 * (e & 7)) : make_double2(0.0, 0.0);
+      }
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int e = e0 + q * NT;
-      if (e < nel) *reinterpret_cast<double2 *>(sb + 2 * e) = v[q];
-    }
+    for (int j = 0; j < CT; ++j)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int e = e0 + q * NT;
+        if (e < nel) *reinterpret_cast<double2 *>(sb + 2 * (j * nel + e)) = v[j][q];
+      }
   }
 }
-
 // A unit's table rows: the lane's value of step s (4 K values) lies `lane`
 // bytes into row group w + s * pitch.  w is the same in all lanes, so a load
 // is a scalar base and one constant lane offset.
@@ -800,9 +800,10 @@ __device__ __forceinline__ void leg_fwd_f64_staged_item(
   unit.chunk(0, table(wave), 0);
   // the Fourier scratch is 16-byte aligned and its column runs are even
   stage_rows<4, NW * 64, CT>(sb, 2 * P2p, [&](int j, int r, int c) {
-    const int par = r >= P2p, p = r - par * P2p, col = (ct0 + j) * 16 + c;
-    return (p < P2 && col < ncol) ? *reinterpret_cast<const double2 *>(four + geo.at(p, m, par, col))
-                                  : make_double2(0.0, 0.0);
+    const int par = r >= P2p, p = r - par * P2p, col = (ct0 + j) * 16;
+    return (p < P2 && col + c < ncol) ? *reinterpret_cast<const double2 *>(
+                                            four + geo.tile(m, col) + (p * geo.pair() + par * geo.parity() + c))
+                                      : make_double2(0.0, 0.0);
   });
   __syncthreads();
   double *__restrict__ sm = spec + (size_t)coef_off(N, m) * ncol;
@@ -883,7 +884,8 @@ __device__ __forceinline__ void leg_inv_f64_staged_item(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int p = rt * 16 + i * 4 + kq;
-          if (p < P2) put_four<NT>(out + geo.at(p, m, slot, col), acc[c][i]);
+          if (p < P2)
+            put_four<NT>(out + geo.tile(m, (ct0 + c) * 16) + (p * geo.pair() + slot * geo.parity() + r16), acc[c][i]);
         }
     }
   }
@@ -999,10 +1001,11 @@ __global__ __launch_bounds__(NW * 64) void leg_fwd_f64_halves_kernel(
   unit.chunk(0, table(0, wave), 0);
   for (int h = 0; h < 2; ++h) {
     if (h) __syncthreads();
-    stage_rows<4, NW * 64, CT>(sb, 2 * H, [&](int j, int r, int c) {
-      const int par = r >= H, p = h * H + (r - par * H), col = (ct0 + j) * 16 + c;
-      return (p < P2 && col < ncol) ? *reinterpret_cast<const double2 *>(four + geo.at(p, m, par, col))
-                                    : make_double2(0.0, 0.0);
+    stage_rows<2, NW * 64, CT>(sb, 2 * H, [&](int j, int r, int c) {
+      const int par = r >= H, p = h * H + (r - par * H), col = (ct0 + j) * 16;
+      return (p < P2 && col + c < ncol) ? *reinterpret_cast<const double2 *>(
+                                              four + geo.tile(m, col) + (p * geo.pair() + par * geo.parity() + c))
+                                        : make_double2(0.0, 0.0);
     });
     __syncthreads();
 #pragma unroll
@@ -1069,7 +1072,7 @@ __global__ __launch_bounds__(NW * 64) void leg_inv_f64_halves_kernel(
     const int slo = h ? S0 : 0, ns = h ? S - S0 : S0, rows = 4 * ns;
     if (ns == 0) break;
     if (h) __syncthreads();
-    stage_rows<4, NW * 64, CT>(sb, 2 * rows, [&](int j, int r, int c) {
+    stage_rows<1, NW * 64, CT>(sb, 2 * rows, [&](int j, int r, int c) {
       const int par = r >= rows, k = 4 * slo + (r - par * rows), col = (ct0 + j) * 16 + c;
       if (k >= (par ? ko : ke) || col >= ncol) return make_double2(0.0, 0.0);
       const double *x = sp + (size_t)(2 * k + par) * ncol + col;
@@ -1097,7 +1100,8 @@ __global__ __launch_bounds__(NW * 64) void leg_inv_f64_halves_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int p = rt * 16 + j * 4 + kq;
-          if (p < P2) put_four<NT>(out + geo.at(p, m, slot, col), acc[i][c][j]);
+          if (p < P2)
+            put_four<NT>(out + geo.tile(m, (ct0 + c) * 16) + (p * geo.pair() + slot * geo.parity() + r16), acc[i][c][j]);
         }
     }
   }
@@ -1134,10 +1138,12 @@ __global__ __launch_bounds__(NW * 64) void leg_fwd_f64_div_kernel(
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
       const int e = threadIdx.x + i * NW * 64, r = e >> 3, par = r >= P2p, p = r - par * P2p;
-      const int c = ct * 16 + 2 * (e & 7);
+      const int c = 2 * (e & 7);
       const double *four = h ? fb : fa;
-      const bool ok = four && r < 2 * P2p && p < P2 && c < ncol;
-      v[h][i] = ok ? *reinterpret_cast<const double2 *>(four + geo.at(p, m, par, c)) : make_double2(0.0, 0.0);
+      const bool ok = four && r < 2 * P2p && p < P2 && ct * 16 + c < ncol;
+      v[h][i] = ok ? *reinterpret_cast<const double2 *>(four + geo.tile(m, ct * 16) +
+                                                        (p * geo.pair() + par * geo.parity() + c))
+                   : make_double2(0.0, 0.0);
     }
   auto table = [&](int h, int u) {  // units past the last: unit 0, loaded but not run
     const int uc = u < 2 * nrt ? u : 0, q = uc & 1, rt = uc >> 1;
