@@ -964,18 +964,17 @@ int inv_staged_launch(const Plan &p, const double *spec, double *four, double *f
   return SHT_OK;
 }
 
-// Staged in two parts: the same shape for large batches on the T170 grid.
-// The K range (latitude pairs for the forward, degree steps of each parity
-// for the inverse) is staged and run in two halves, so the LDS block of half
-// the K range holds more column tiles -- two for the forward, four for the
-// inverse -- and each table fragment feeds that many MFMAs.  The steps of an
-// output tile still run in order from a zero accumulator, so results are
-// bitwise those of the one-part kernels; a wave's MAXU units keep their
-// accumulators across the halves and store after the second.  Measured at
-// T170 (eight waves): 776 fields forward 261 against 280 us, inverse 234
-// against 254 us; 388 fields 144 / 136.5 against 148 / 143.5 us; at 97 fields
-// slower (37-40 against 34-39 us), hence the batch threshold at dispatch.
-// Forward: LDS [CT][parity][P2p / 2 pairs][16].
+// Staged in two parts: the forward for larger batches on the T170 grid.  The
+// latitude pairs are staged and run in two halves, so the LDS block of half of
+// them holds two column tiles and each table value feeds two MFMAs.  The steps
+// of an output tile still run in order from a zero accumulator, so results are
+// bitwise those of the one-part kernel; a wave's MAXU units keep their
+// accumulators across the halves and store after the second.  Measured at T170
+// (eight waves), one part / two: 33 fields 16.1 / 16.0 us, 97 fields 36.5 / 34.4,
+// 145 fields 50.2 / 46.5, 388 fields 133 / 123, 776 fields 267 / 237.  (The
+// inverse, whose two-tile block fits whole, gains nothing: with four tiles 388
+// fields 119 against 113 us, 776 fields 218 against 206.)
+// LDS [CT][parity][P2p / 2 pairs][16].
 template <int CT, int D, int NW, int MAXU>
 __global__ __launch_bounds__(NW * 64) void leg_fwd_f64_halves_kernel(
     const double *__restrict__ four, double *__restrict__ spec, const double *__restrict__ Pfwd,
@@ -1031,77 +1030,6 @@ __global__ __launch_bounds__(NW * 64) void leg_fwd_f64_halves_kernel(
         for (int j = 0; j < 4; ++j) {
           const int k = rt * 16 + j * 4 + kq;
           if (k < kn) put_spec(sm + (size_t)(2 * k + q) * ncol + col, acc[i][c][j]);
-        }
-    }
-  }
-}
-
-// Inverse: steps S = KP / 4 of each parity split S0 = ceil(S / 2) + the rest;
-// LDS [CT][parity][4 S0 rows][16].
-template <int CT, int D, int NW, int MAXU, bool NT>
-__global__ __launch_bounds__(NW * 64) void leg_inv_f64_halves_kernel(
-    const double *__restrict__ spec, double *__restrict__ four, double *__restrict__ four2,
-    const double *__restrict__ Pinv, const double *__restrict__ Hinv, const int *__restrict__ poff,
-    const int *__restrict__ mlist, int mlen, int N, int P2, int P2p, int ncol, int nct, int tab0,
-    int ntab, FourGeom geo) {
-  extern __shared__ double sb[];
-  const int ncg = (nct + CT - 1) / CT;
-  int m, t;
-  if (!xcd_m_block(blockIdx.x, mlist, mlen, ntab * ncg, m, t)) return;
-  const int tab = tab0 + t % ntab, ct0 = (t / ntab) * CT;
-  const int nn = N - m + 1, ke = (nn + 1) >> 1, ko = nn >> 1;
-  const int KP = (ke + 3) & ~3, S = KP >> 2, S0 = (S + 1) >> 1;
-  const double *__restrict__ sp = spec + (size_t)coef_off(N, m) * ncol;
-  const int wave = wave_id(), lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
-  const int rtiles = P2p >> 4;
-  double *__restrict__ out = tab ? four2 : four;
-  const int se = tab ? 1 : 0;  // the derivative table's parities are swapped
-  d4 acc[MAXU][CT];
-#pragma unroll
-  for (int i = 0; i < MAXU; ++i)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[i][c] = d4{0.0, 0.0, 0.0, 0.0};
-  auto table = [&](int h, int u) {  // an empty second half: the first again, loaded but not run
-    const int uc = u < 2 * rtiles ? u : 0, q = uc & 1, rt = uc >> 1, hc = S > S0 ? h : 0;
-    return TableCol{(tab ? Hinv : Pinv) + poff[m] + ((size_t)q * KP + 4 * hc * S0) * P2p + rt * 16,
-                    (kq * P2p + r16) * 8u, 4u * P2p, hc ? S - S0 : S0};
-  };
-  StagedUnit<CT, D> unit;
-  unit.chunk(0, table(0, wave), 0);
-  for (int h = 0; h < 2; ++h) {
-    const int slo = h ? S0 : 0, ns = h ? S - S0 : S0, rows = 4 * ns;
-    if (ns == 0) break;
-    if (h) __syncthreads();
-    stage_rows<1, NW * 64, CT>(sb, 2 * rows, [&](int j, int r, int c) {
-      const int par = r >= rows, k = 4 * slo + (r - par * rows), col = (ct0 + j) * 16 + c;
-      if (k >= (par ? ko : ke) || col >= ncol) return make_double2(0.0, 0.0);
-      const double *x = sp + (size_t)(2 * k + par) * ncol + col;
-      return make_double2(x[0], x[1]);
-    });
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < MAXU; ++i) {
-      const int u = wave + NW * i, q = u & 1, un = u + NW;
-      if (u >= 2 * rtiles) break;
-      const bool last = i + 1 == MAXU || un >= 2 * rtiles;  // of this half
-      const double *B = sb + (q * rows + kq) * 16 + r16;
-      unit.run(table(h, u), last ? table(1, wave) : table(h, un), B, 2 * rows * 16, acc[i]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < MAXU; ++i) {
-    const int u = wave + NW * i, q = u & 1, rt = u >> 1;
-    if (u >= 2 * rtiles) break;
-    const int slot = q ^ se;
-#pragma unroll
-    for (int c = 0; c < CT; ++c) {
-      const int col = (ct0 + c) * 16 + r16;
-      if (col < ncol)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int p = rt * 16 + j * 4 + kq;
-          if (p < P2)
-            put_four<NT>(out + geo.tile(m, (ct0 + c) * 16) + (p * geo.pair() + slot * geo.parity() + r16), acc[i][c][j]);
         }
     }
   }
@@ -1220,11 +1148,10 @@ int f64_multi_launch(const MultiGroup *g, int n, hipStream_t s) {
   return SHT_OK;
 }
 
-// Field count from which the staged shape runs in two parts on the T170 grid.
-constexpr int kHalvesMinFields = 192;
+// Field count from which the staged forward runs in two parts on the T170 grid.
+constexpr int kHalvesMinFields = 64;
 
-// MAXU = 2: at most 2 nrt(0) <= 16 forward units, and 2 (P2p / 16) = 16
-// inverse units at P2p = 128, over eight waves.
+// MAXU = 2: at most 2 nrt(0) <= 16 forward units over eight waves.
 template <int CT, int MAXU>
 int fwd_halves_launch(const Plan &p, const double *four, double *spec, int nf, hipStream_t s) {
   const int ncol = 2 * nf, nct = (ncol + 15) / 16;
@@ -1235,21 +1162,6 @@ int fwd_halves_launch(const Plan &p, const double *four, double *spec, int nf, h
   SHT_HIP(hipGetLastError());
   return SHT_OK;
 }
-template <int CT, int MAXU>
-int inv_halves_launch(const Plan &p, const double *spec, double *four, double *four2, int tab0,
-                      int ntab, int nf, hipStream_t s) {
-  const int ncol = 2 * nf, nct = (ncol + 15) / 16;
-  const int S = roundup(ceil_half(p.N + 1), 4) / 4, S0 = (S + 1) / 2;
-  const size_t lds = sizeof(double) * ((CT * 2 - 1) * 4 * S0 + roundup(4 * S0, 16)) * 16;
-  const FourGeom geo = four_geom_out(p, nf, sizeof(double));
-  launch_kernel(geo.stream ? leg_inv_f64_halves_kernel<CT, 4, 8, MAXU, true>
-                           : leg_inv_f64_halves_kernel<CT, 4, 8, MAXU, false>,
-      xcd_m_blocks(p, 0, ntab * ((nct + CT - 1) / CT)), 512, lds, s, spec, four, four2, p.Pinv, p.Hinv,
-      p.poff_inv, p.xcd_m[0], p.xcd_mlen[0], p.N, p.P2, p.P2p, ncol, nct, tab0, ntab, geo);
-  SHT_HIP(hipGetLastError());
-  return SHT_OK;
-}
-
 template <int RT>
 int inv_launch(const Plan &p, const double *spec, double *four, double *four2, int tab0, int ntab,
                int nf, hipStream_t s) {
@@ -1347,9 +1259,6 @@ int launch_leg_inv_f64_shape(const Plan &p, int shape, const double *spec, doubl
   const int tab0 = value_table ? 0 : 1;
   const int ntab = (value_table && deriv_table) ? 2 : 1;
   if (shape == SHT_SHAPE_WAVE) return inv_wave_launch<4>(p, spec, four, four2, tab0, ntab, nf, s);
-  // two-part staging for large batches on the 128-pair grid (T170)
-  if (shape == SHT_SHAPE_STAGED && p.P2p == 128 && nf >= kHalvesMinFields)
-    return inv_halves_launch<4, 2>(p, spec, four, four2, tab0, ntab, nf, s);
   if (shape == SHT_SHAPE_STAGED)
     return p.P2p >= 128 ? inv_staged_launch<2, 8>(p, spec, four, four2, tab0, ntab, nf, s)
                         : inv_staged_launch<1, 4>(p, spec, four, four2, tab0, ntab, nf, s);
