@@ -665,8 +665,8 @@ int fwd_wave_launch(const Plan &p, const double *four, double *spec, int nf, hip
 //
 // NW waves share the block: from P2p = 128 latitude pairs (the T170 grid)
 // eight, and the inverse there takes two column tiles (each table fragment
-// feeds two MFMAs, halving the table traffic from L2); below that four waves
-// and one column tile.  Measured at T170, 776 fields: inverse 248 against
+// feeds two MFMAs, halving the table traffic from L2) except in small calls
+// (kOneTileMaxFields); below that four waves and one column tile.  Measured at T170, 776 fields: inverse 248 against
 // 273 us with four waves and one tile, forward 277 against 295 us (two tiles
 // for the forward: 276 us, but slower at 97 and 388 fields); eight waves were
 // slower at T42 and T85.  Measured no faster: table loads 8 or 16 steps
@@ -1148,6 +1148,17 @@ int f64_multi_launch(const MultiGroup *g, int n, hipStream_t s) {
   return SHT_OK;
 }
 
+// Field count up to which the staged inverse of one table takes one column tile
+// per workgroup on the T170 grid.  Two tiles halve the table reads, but their
+// half as many workgroups (684 for 33 to 64 fields) leave the chip's last wave
+// part empty: one / two tiles, Legendre step, 32 fields 12.1 / 13.7 us, 40 fields
+// 15.5 / 17.6, 56 fields 19.2 / 21.1, 57 and 64 fields equal, 80 fields 29.2 / 27.3,
+// 145 fields 57.2 / 50.1.  With both tables (gradients) the workgroups are twice
+// as many and two tiles win from 32 fields on (24.3 / 23.2), as they do on grids
+// of more latitude pairs (N = 200, 40 fields 25.1 / 23.5).  Either way each output
+// tile runs the same products in the same order: the results are the same.
+constexpr int kOneTileMaxFields = 56;
+
 // Field count from which the staged forward runs in two parts on the T170 grid.
 constexpr int kHalvesMinFields = 64;
 
@@ -1259,9 +1270,12 @@ int launch_leg_inv_f64_shape(const Plan &p, int shape, const double *spec, doubl
   const int tab0 = value_table ? 0 : 1;
   const int ntab = (value_table && deriv_table) ? 2 : 1;
   if (shape == SHT_SHAPE_WAVE) return inv_wave_launch<4>(p, spec, four, four2, tab0, ntab, nf, s);
-  if (shape == SHT_SHAPE_STAGED)
-    return p.P2p >= 128 ? inv_staged_launch<2, 8>(p, spec, four, four2, tab0, ntab, nf, s)
-                        : inv_staged_launch<1, 4>(p, spec, four, four2, tab0, ntab, nf, s);
+  if (shape == SHT_SHAPE_STAGED) {
+    if (p.P2p < 128) return inv_staged_launch<1, 4>(p, spec, four, four2, tab0, ntab, nf, s);
+    if (p.P2p == 128 && ntab == 1 && nf <= kOneTileMaxFields)
+      return inv_staged_launch<1, 8>(p, spec, four, four2, tab0, ntab, nf, s);
+    return inv_staged_launch<2, 8>(p, spec, four, four2, tab0, ntab, nf, s);
+  }
   if (shape == SHT_SHAPE_TILE || shape == SHT_SHAPE_TILE_SPLIT) {
     const int rtiles = p.P2p / 16;
     int rt = 4;

@@ -364,3 +364,18 @@ def test_mixed_streaming_shapes_bitwise(prec, N, im, jm, nf):
     p.set_shapes(nf, shtamd.SHAPE_STAGED, shtamd.SHAPE_TILE)
     assert np.array_equal(run_inverse(p, spec, nf)[0], g0) and np.array_equal(run_forward(p, grid, nf), s0)
     p.close()
+
+
+@pytest.mark.parametrize("N,im,jm,nf", [(170, 512, 256, 33), (170, 512, 256, 56), (170, 512, 256, 57), (113, 512, 242, 1), (10, 512, 256, 50)])
+def test_staged_inverse_column_tiles_bitwise(N, im, jm, nf):
+    """The staged inverse of the 128-pair grids with one and with two column tiles
+    per workgroup (up to 56 fields, above), value and gradient tables: bitwise WAVE."""
+    spec = synth.spectra(N, nf, cfg=11)
+    p = shtamd.Plan(N, im, jm, nf, flags=shtamd.FLAG_GRAD)
+    got = []
+    for shape in (shtamd.SHAPE_WAVE, shtamd.SHAPE_STAGED):
+        p.set_shapes(nf, shape, shtamd.SHAPE_AUTO)
+        got.append(run_inverse(p, spec, nf))
+        got[-1] += run_inverse(p, spec, nf, grad=True)
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    p.close()
