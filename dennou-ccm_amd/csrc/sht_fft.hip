@@ -11,7 +11,7 @@
 //   inverse:  from the Legendre sums E (even n-m) and O (odd): X_N = E + O,
 //             X_S = E - O, Z_m = X_N + i X_S, Z_{L-m} = conj X_N + i conj X_S,
 //             z = IFFT(Z): f_N = Re z, f_S = Im z.
-// The Fourier coefficients are read/written in the [pair][m][parity][field]
+// The Fourier coefficients are read/written in the [group][pair][m][parity][field]
 // layout the Legendre GEMMs want, so this kernel is also the (lat,lon) <->
 // (m,lat) transpose: global traffic is row-contiguous on the grid side and
 // runs of 2G values on the Fourier side; the reordering happens in LDS.

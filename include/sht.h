@@ -350,8 +350,8 @@ enum {
   SHT_SHAPE_STAGED = 4,       /* FP64: workgroup per (m, 16 columns), data block in LDS,
                                  each wave a (parity, row tile) over the whole K; mixed
                                  inverse on grids of <= 128 latitude pairs: workgroup per
-                                 (m, 8 column tiles), the table held in registers while
-                                 the spectral tiles stream through LDS                   */
+                                 (m, up to 16 column tiles), the table held in registers
+                                 while the spectral tiles stream through LDS                   */
   SHT_SHAPE_FUSED = 5,        /* inverse of mixed plans with 64 <= im <= 512 and
                                  nmax < 192: KSPLIT's Legendre items and the ring FFTs
                                  in one persistent launch (grid values; gradients and
@@ -363,7 +363,9 @@ enum {
  * plans take SHT_SHAPE_AUTO, SHT_SHAPE_KSPLIT (workgroup per (m, 16 columns),
  * data tile shared in LDS), SHT_SHAPE_WAVE (wavefront per 16 columns, data
  * tile in registers) and SHT_SHAPE_TILE (workgroup per (m, 32 columns), each
- * wave's table fragments used for both column tiles), and for the inverse
+ * wave's table fragments used for both column tiles; the forward on grids of
+ * 113 to 128 latitude pairs streams the data tiles past a table held in
+ * registers where that is faster), and for the inverse
  * SHT_SHAPE_STAGED (jm <= 256) and SHT_SHAPE_FUSED where the plan has them
  * (SHT_ERR_UNSUPPORTED otherwise); their results are bitwise equal. */
 int sht_plan_set_shapes(sht_plan *plan, int nf, int inv_shape, int fwd_shape);
