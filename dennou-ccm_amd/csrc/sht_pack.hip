@@ -110,14 +110,20 @@ __global__ __launch_bounds__(256) void canon_to_spml_kernel(const double *__rest
 }
 
 // one block per field: (1/4pi) sum_ij (2pi/im) w_j f_ij.  One CU reads a whole
-// field, so the kernel is bound by what that CU has in flight: every thread
-// issues kAvrAhead 16-byte loads before it adds the first (W = 2 values; W = 1
-// for a grid that is only 8-byte aligned), and the block is as wide as the
-// field allows (avr_threads).  12 fields of 256 x 128: 37.9 -> 5.7 us (256
-// threads, one load at a time before); with 8-byte loads 9.8 us.  A pair never
-// straddles a row: im is even.
-constexpr int kAvrAhead = 8;
-template <int W>
+// field, so the kernel is bound by what that CU has in flight and by its load
+// instructions: every thread issues kAvrAhead 16-byte loads before it adds the
+// first (W = 2 values; W = 1 for a grid that is only 8-byte aligned), and the
+// block is as wide as the field allows (avr_threads).  LONG, for fields of more
+// than one such round of a full block: the next round's loads are in flight
+// while one is added, and the row weights come from LDS instead of a second
+// load per pair; a thread adds the same values in the same order either way.
+// 12 fields of 256 x 128: 6.1 -> 4.9 us (37.9 with 256 threads and one load at a
+// time), 97 fields 7.1 -> 6.6, one field of 512 x 256 16.9 -> 10.4; 8-byte
+// loads 6.9 us at 12 fields.  Fields of one round gain nothing from it and pay
+// the barrier (128 x 64, 26 fields 3.3 against 3.6 us).  A pair never straddles a
+// row: im is even.
+constexpr int kAvrAhead = 8, kAvrMaxRows = 512;
+template <int W, bool LONG>
 __global__ __launch_bounds__(1024) void avr_kernel(const double *__restrict__ grid,
                                                    const double *__restrict__ w,
                                                    double *__restrict__ avg, int im, int lim, int n) {
@@ -125,20 +131,43 @@ __global__ __launch_bounds__(1024) void avr_kernel(const double *__restrict__ gr
   const int f = blockIdx.x, step = blockDim.x * W;
   const double *__restrict__ g = grid + (size_t)f * n;
   double acc = 0.0;
-  for (int t0 = threadIdx.x * W; t0 < n; t0 += kAvrAhead * step) {
-    vec v[kAvrAhead];
-    double wj[kAvrAhead];
+  auto load = [&](int t0, vec (&v)[kAvrAhead]) {
 #pragma unroll
     for (int q = 0; q < kAvrAhead; ++q) {
-      const int t = t0 + q * step, c = t < n ? t : t0;  // past the end: a valid address, not added
-      v[q] = *reinterpret_cast<const vec *>(g + c);
-      wj[q] = w[c >> lim];
+      const int t = t0 + q * step;
+      v[q] = *reinterpret_cast<const vec *>(g + (t < n ? t : 0));  // past the end: a valid address, not added
     }
+  };
+  auto add = [&](int t0, const vec (&v)[kAvrAhead], auto weight) {
 #pragma unroll
     for (int q = 0; q < kAvrAhead; ++q)
       if (t0 + q * step < n)
 #pragma unroll
-        for (int i = 0; i < W; ++i) acc += wj[q] * v[q][i];
+        for (int i = 0; i < W; ++i) acc += weight(q) * v[q][i];
+  };
+  int t0 = threadIdx.x * W;
+  if constexpr (LONG) {
+    __shared__ double ws[kAvrMaxRows];
+    vec a[kAvrAhead], b[kAvrAhead];
+    load(t0, a);
+    for (int j = threadIdx.x; j < n >> lim; j += blockDim.x) ws[j] = w[j];
+    __syncthreads();
+    for (; t0 < n; t0 += 2 * kAvrAhead * step) {
+      const int t1 = t0 + kAvrAhead * step, t2 = t1 + kAvrAhead * step;
+      load(t1, b);
+      add(t0, a, [&](int q) { return ws[(t0 + q * step) >> lim]; });
+      if (t2 < n) load(t2, a);
+      add(t1, b, [&](int q) { return ws[(t1 + q * step) >> lim]; });
+    }
+  } else {
+    for (; t0 < n; t0 += kAvrAhead * step) {
+      vec v[kAvrAhead];
+      double wj[kAvrAhead];
+      load(t0, v);
+#pragma unroll
+      for (int q = 0; q < kAvrAhead; ++q) wj[q] = w[(t0 + q * step < n ? t0 + q * step : t0) >> lim];
+      add(t0, v, [&](int q) { return wj[q]; });
+    }
   }
 #pragma unroll
   for (int s = 32; s > 0; s >>= 1) acc += __shfl_xor(acc, s);
@@ -228,7 +257,9 @@ int launch_canon_to_spml(const Plan &p, const double *spec, double *wa, int nf, 
 
 int launch_avr_lonlat(const Plan &p, const double *grid, double *avg, int nf, hipStream_t s) {
   const int n = p.im * p.jm;
-  const auto kern = ((uintptr_t)grid & 15) == 0 ? avr_kernel<2> : avr_kernel<1>;
+  const bool two = ((uintptr_t)grid & 15) == 0, lng = n > 2 * kAvrAhead * 1024;
+  const auto kern = two ? (lng ? avr_kernel<2, true> : avr_kernel<2, false>)
+                        : (lng ? avr_kernel<1, true> : avr_kernel<1, false>);
   kern<<<nf, avr_threads(n), 0, s>>>(grid, p.w, avg, p.im, __builtin_ctz(p.im), n);
   SHT_HIP(hipGetLastError());
   return SHT_OK;

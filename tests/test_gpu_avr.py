@@ -25,3 +25,11 @@ def test_avr_against_oracle(N, im, jm, shift):
     # im jm terms of size 200 summed in another order: 512 x 256 of them stay within 2e-12 of each other
     assert np.abs(avg.cpu().numpy() - oracle.Plan(N, im, jm).avr_lonlat(g)).max() < 2e-12
     p.close()
+
+
+@pytest.mark.parametrize("N,im,jm", [(40, 256, 64), (40, 256, 66), (5, 256, 512), (5, 1024, 126), (60, 2048, 62)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_avr_of_several_rounds(N, im, jm, shift):
+    """Fields of one full round and a little more, of a part-filled last round, of
+    the most rows: against the oracle, at most 512 x 256 terms as above."""
+    test_avr_against_oracle(N, im, jm, shift)
