@@ -839,21 +839,23 @@ __global__ __launch_bounds__(NW * 64) void leg_fwd_f64_staged_kernel(
   leg_fwd_f64_staged_item<CT, D, NW>(sb, four, spec, Pfwd, poff, N, P2, P2p, ncol, geo, m, t);
 }
 
-// Inverse, workgroup = (m, table, CT column tiles); LDS [CT][parity][KP][16]
+// Inverse, workgroup = (m, table or tables, CT column tiles); LDS [CT][parity][KP][16]
 // with KP = this m's degrees per parity rounded up to 4 (rows past a parity's
 // last degree hold zeros).
-template <int CT, int D, int NW, bool NT>
+// MERGE: both tables, the value table's units first; else table tab0.
+template <int CT, int D, int NW, bool NT, bool MERGE>
 __device__ __forceinline__ void leg_inv_f64_staged_item(
     double *sb, const double *__restrict__ spec, double *__restrict__ four, double *__restrict__ four2,
     const double *__restrict__ Pinv, const double *__restrict__ Hinv, const int *__restrict__ poff, int N, int P2,
-    int P2p, int ncol, FourGeom geo, int m, int tab, int ct0) {
+    int P2p, int ncol, FourGeom geo, int m, int tab0, int ct0) {
   const int nn = N - m + 1, ke = (nn + 1) >> 1, ko = nn >> 1;
   const int KP = (ke + 3) & ~3;
   const double *__restrict__ sp = spec + (size_t)coef_off(N, m) * ncol;
   const int wave = wave_id(), lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
-  const int rtiles = P2p >> 4;
+  const int half = P2p >> 3, nunits = MERGE ? 2 * half : half;  // a table's units: 2 parities x 16-row tiles
   auto table = [&](int u) {  // units past the last: unit 0, loaded but not run
-    const int uc = u < 2 * rtiles ? u : 0, q = uc & 1, rt = uc >> 1;
+    const int uc = u < nunits ? u : 0, second = MERGE && uc >= half, tab = MERGE ? second : tab0, q = uc & 1,
+              rt = (second ? uc - half : uc) >> 1;
     return TableCol{(tab ? Hinv : Pinv) + poff[m] + (size_t)q * KP * P2p + rt * 16, (kq * P2p + r16) * 8u, 4u * P2p,
                     KP >> 2};
   };
@@ -867,10 +869,10 @@ __device__ __forceinline__ void leg_inv_f64_staged_item(
     return make_double2(x[0], x[1]);
   });
   __syncthreads();
-  double *__restrict__ out = tab ? four2 : four;
-  const int se = tab ? 1 : 0;  // the derivative table's parities are swapped
-  for (int u = wave; u < 2 * rtiles; u += NW) {
-    const int q = u & 1, rt = u >> 1;
+  for (int u = wave; u < nunits; u += NW) {
+    const int second = MERGE && u >= half, tab = MERGE ? second : tab0, q = u & 1, rt = (second ? u - half : u) >> 1;
+    double *__restrict__ out = tab ? four2 : four;
+    const int se = tab ? 1 : 0;  // the derivative table's parities are swapped
     const double *B = sb + (q * KP + kq) * 16 + r16;
     d4 acc[CT];
 #pragma unroll
@@ -891,7 +893,7 @@ __device__ __forceinline__ void leg_inv_f64_staged_item(
   }
 }
 
-template <int CT, int D, int NW, bool NT>
+template <int CT, int D, int NW, bool NT, bool MERGE>
 __global__ __launch_bounds__(NW * 64) void leg_inv_f64_staged_kernel(
     const double *__restrict__ spec, double *__restrict__ four, double *__restrict__ four2,
     const double *__restrict__ Pinv, const double *__restrict__ Hinv, const int *__restrict__ poff,
@@ -900,9 +902,10 @@ __global__ __launch_bounds__(NW * 64) void leg_inv_f64_staged_kernel(
   extern __shared__ double sb[];
   const int ncg = (nct + CT - 1) / CT;
   int m, t;
-  if (!xcd_m_block(blockIdx.x, mlist, mlen, ntab * ncg, m, t)) return;
-  leg_inv_f64_staged_item<CT, D, NW, NT>(sb, spec, four, four2, Pinv, Hinv, poff, N, P2, P2p, ncol, geo, m,
-                                         tab0 + t % ntab, (t / ntab) * CT);
+  const int per = MERGE ? 1 : ntab;  // workgroups per column group
+  if (!xcd_m_block(blockIdx.x, mlist, mlen, per * ncg, m, t)) return;
+  leg_inv_f64_staged_item<CT, D, NW, NT, MERGE>(sb, spec, four, four2, Pinv, Hinv, poff, N, P2, P2p, ncol, geo, m,
+                                         tab0 + t % per, (t / per) * CT);
 }
 
 // ---- Several groups in one launch (sht_internal.h, MultiGroup): the staged
@@ -928,7 +931,7 @@ __global__ __launch_bounds__(256) void leg_f64_multi_kernel(F64Multi a) {
   if constexpr (FWD)
     leg_fwd_f64_staged_item<1, 4, 4>(sb, g.four, g.spec_out, g.table, g.poff, g.N, g.P2, g.P2p, g.ncol, g.geo, m, t);
   else
-    leg_inv_f64_staged_item<1, 4, 4, NT>(sb, g.spec_in, g.four, nullptr, g.table, nullptr, g.poff, g.N, g.P2, g.P2p,
+    leg_inv_f64_staged_item<1, 4, 4, NT, false>(sb, g.spec_in, g.four, nullptr, g.table, nullptr, g.poff, g.N, g.P2, g.P2p,
                                          g.ncol, g.geo, m, 0, t);
 }
 
@@ -956,9 +959,20 @@ int inv_staged_launch(const Plan &p, const double *spec, double *four, double *f
                       int ntab, int nf, hipStream_t s) {
   const int ncol = 2 * nf, nct = (ncol + 15) / 16;
   const FourGeom geo = four_geom_out(p, nf, sizeof(double));
-  launch_kernel(geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true>
-                           : leg_inv_f64_staged_kernel<CT, 4, NW, false>,
-      xcd_m_blocks(p, 0, ntab * ((nct + CT - 1) / CT)), NW * 64, inv_staged_lds(p, CT), s, spec, four, four2, p.Pinv, p.Hinv,
+  // both tables in one workgroup: the spectra are staged once, but half as many
+  // workgroups run twice as long, so only where those fill the chip (2048 are two
+  // rounds of four per CU), or half as many if a wave has one unit per table and
+  // the staging is most of a workgroup's life.  Gradients' Legendre step, one
+  // table / both per workgroup: T21 400 fields 6.6 / 6.0 us; T42 79 fields 5.8 / 5.7,
+  // 192 fields 7.9 / 6.8, 388 fields 13.1 / 10.6; T85 97 fields 12.0 / 12.6, 190 fields
+  // 23.8 / 22.0; T170 64 fields 40.8 / 44.9, 192 fields 111 / 107.
+  const int nwg = xcd_m_blocks(p, 0, (nct + CT - 1) / CT);
+  const bool merge = ntab == 2 && nwg >= (p.P2p / 8 <= NW ? 1024 : 2048);
+  launch_kernel(merge ? (geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true, true>
+                                    : leg_inv_f64_staged_kernel<CT, 4, NW, false, true>)
+                      : (geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true, false>
+                                    : leg_inv_f64_staged_kernel<CT, 4, NW, false, false>),
+      merge ? nwg : xcd_m_blocks(p, 0, ntab * ((nct + CT - 1) / CT)), NW * 64, inv_staged_lds(p, CT), s, spec, four, four2, p.Pinv, p.Hinv,
       p.poff_inv, p.xcd_m[0], p.xcd_mlen[0], p.N, p.P2, p.P2p, ncol, nct, tab0, ntab, geo);
   SHT_HIP(hipGetLastError());
   return SHT_OK;

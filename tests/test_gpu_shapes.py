@@ -379,3 +379,17 @@ def test_staged_inverse_column_tiles_bitwise(N, im, jm, nf):
         got[-1] += run_inverse(p, spec, nf, grad=True)
     assert all(np.array_equal(a, b) for a, b in zip(*got))
     p.close()
+
+
+@pytest.mark.parametrize("N,im,jm,nf", [(42, 128, 64, 185), (42, 128, 64, 184), (10, 32, 16, 800), (85, 256, 128, 190), (170, 512, 256, 195)])
+def test_staged_gradients_both_tables_bitwise(N, im, jm, nf):
+    """The staged inverse with both tables in one workgroup and with one each, on both
+    sides of the line: bitwise WAVE."""
+    spec = synth.spectra(N, nf, cfg=12)
+    p = shtamd.Plan(N, im, jm, nf, flags=shtamd.FLAG_GRAD)
+    got = []
+    for shape in (shtamd.SHAPE_WAVE, shtamd.SHAPE_STAGED):
+        p.set_shapes(nf, shape, shtamd.SHAPE_AUTO)
+        got.append(run_inverse(p, spec, nf, grad=True))
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    p.close()
