@@ -231,20 +231,34 @@ int zonal_waves(int nsteps) {
   return nw < kZonalMaxWaves ? nw : kZonalMaxWaves;
 }
 
-int zonal_fwd(const sht_zonal *z, const double *y, double *l, int nf, hipStream_t s) {
-  const int nrt = z->KR / 16, nct = (nf + 15) / 16, nw = zonal_waves(z->P2p / 4);
-  zonal_fwd_kernel<<<2 * nrt * nct, 64 * nw, sizeof(double) * 256 * nw, s>>>(
-      y, l, z->Tfwd, z->N, z->jm, z->P2, z->P2p, z->KR, nrt, nf);
-  SHT_HIP(hipGetLastError());
+// Runs launch(first field, fields, workgroups) over ranges of fields that keep
+// each launch below 2^32 threads (the runtime's limit of a grid dimension), at
+// `tiles` workgroups of nw waves per 16 fields.  Only calls of some 2^31 values reach it.
+template <class Launch>
+int zonal_ranges(int nf, int tiles, int nw, Launch launch) {
+  const int64_t most = 16 * (int64_t)(UINT32_MAX / (64u * nw) / tiles);
+  for (int64_t f0 = 0; f0 < nf; f0 += most) {
+    const int n = (int)(nf - f0 < most ? nf - f0 : most);
+    launch(f0, n, tiles * ((n + 15) / 16));
+    SHT_HIP(hipGetLastError());
+  }
   return SHT_OK;
 }
 
+int zonal_fwd(const sht_zonal *z, const double *y, double *l, int nf, hipStream_t s) {
+  const int nrt = z->KR / 16, nw = zonal_waves(z->P2p / 4);
+  return zonal_ranges(nf, 2 * nrt, nw, [&](int64_t f0, int n, int wgs) {
+    zonal_fwd_kernel<<<wgs, 64 * nw, sizeof(double) * 256 * nw, s>>>(
+        y + f0 * z->jm, l + f0 * (z->N + 1), z->Tfwd, z->N, z->jm, z->P2, z->P2p, z->KR, nrt, n);
+  });
+}
+
 int zonal_inv(const sht_zonal *z, const double *l, double *y, int nf, hipStream_t s) {
-  const int nrt = z->P2p / 16, nct = (nf + 15) / 16, nw = zonal_waves(2 * (z->KP / 4));
-  zonal_inv_kernel<<<nrt * nct, 64 * nw, sizeof(double) * 256 * nw, s>>>(
-      l, y, z->Tinv, z->N, z->jm, z->P2, z->P2p, z->KP, nrt, nf);
-  SHT_HIP(hipGetLastError());
-  return SHT_OK;
+  const int nrt = z->P2p / 16, nw = zonal_waves(2 * (z->KP / 4));
+  return zonal_ranges(nf, nrt, nw, [&](int64_t f0, int n, int wgs) {
+    zonal_inv_kernel<<<wgs, 64 * nw, sizeof(double) * 256 * nw, s>>>(
+        l + f0 * (z->N + 1), y + f0 * z->jm, z->Tinv, z->N, z->jm, z->P2, z->P2p, z->KP, nrt, n);
+  });
 }
 
 // Synchronous host call through pinned staging: dir 0 = l_y, 1 = y_l.

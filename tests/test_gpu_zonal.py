@@ -110,3 +110,30 @@ def test_zonal_waves_per_tile(nm, jm, nf):
     assert np.linalg.norm(yo - y_ref) / np.linalg.norm(y_ref) < 1e-12
     assert np.array_equal(z.l_y(y[-1]), lo[-1]) and np.array_equal(z.y_l(l[-1]), yo[-1])
     z.close()
+
+
+@pytest.mark.parametrize("nm,jm,nf", [(1024, 1024, 1016802 + 33), (1, 2, (1 << 29) + 33)])
+def test_zonal_calls_beyond_one_launch(nm, jm, nf):
+    """More workgroups than one launch may have (2^32 threads; l_y at degree 1024, both
+    ways on two latitudes): every field is written, and as in a small call."""
+    z = shtamd.Zonal(nm, jm, kmax=nf)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    y = torch.empty((nf, jm), dtype=torch.float64, device="cuda").normal_(generator=gen)
+    l = torch.full((nf, nm + 1), float("nan"), dtype=torch.float64, device="cuda")
+    z.l_y_dev(y, l, nf)
+    assert not any(bool(torch.isnan(c).any()) for c in l.split(1 << 24))
+    back = y[:1].new_full((nf, jm), float("nan")) if jm == 2 else None
+    if back is not None:
+        z.y_l_dev(l, back, nf)
+        assert not any(bool(torch.isnan(c).any()) for c in back.split(1 << 24))
+    # around multiples of 16 fields where a launch may end, and the ends of the call
+    for f0 in (0, nf // 4, nf // 2 - 8, nf - 66, nf - 17):
+        n = min(17, nf - f0)
+        lo = torch.empty((n, nm + 1), dtype=torch.float64, device="cuda")
+        z.l_y_dev(y[f0:f0 + n].clone(), lo, n)
+        assert torch.equal(lo, l[f0:f0 + n]), f0
+        if back is not None:
+            yo = torch.empty((n, jm), dtype=torch.float64, device="cuda")
+            z.y_l_dev(lo, yo, n)
+            assert torch.equal(yo, back[f0:f0 + n]), f0
+    z.close()
