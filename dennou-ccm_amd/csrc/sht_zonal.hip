@@ -67,8 +67,11 @@ __global__ void zonal_table_kernel(int N, int P2, int P2p, int KP, int KR, const
 // are added in wave order in FP64.  Bound by latency: one tile's K loop run by
 // a single wave is a chain of load-MFMA steps, and a one-field call of degree
 // 1024 has only 33-66 tiles.  Measured at nmax = jm = 1024, one field: l_y
-// 32.9 -> 5.5 us, y_l 61.2 -> 7.5 us (the tables are 4.3 MB each; 20 steps
-// ahead for y_l, one round of loads: 9.3 us).
+// 32.9 -> 5.6 us, y_l 61.2 -> 7.1 us (the tables are 4.3 MB each; 20 steps
+// ahead for y_l, one round of loads: 9.3 us).  Only the steps that a wave has
+// are loaded: with their places in a round filled by repeated loads l_y on 32
+// latitudes took 3.4 instead of 2.7 us at 97 fields and 8.4 instead of 4.7 at 5000
+// (one wave a tile: 2.8 and 4.3).
 // nw depends on the plan alone, so a field's result does not depend on nf.
 constexpr int kZonalAhead = 8;
 constexpr int kZonalMaxWaves = 16;
@@ -97,25 +100,33 @@ __global__ __launch_bounds__(64 * kZonalMaxWaves) void zonal_fwd_kernel(
   const double *__restrict__ yf = y + (size_t)(f < nf ? f : 0) * jm;
   const double sgn = q ? -1.0 : 1.0;
   const int nsteps = P2p >> 2;
-  d4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int s0 = wave; s0 < nsteps; s0 += nw * kZonalAhead) {
-    // steps past the end and pairs past P2 load valid addresses and count as 0
-    double a[kZonalAhead], yn[kZonalAhead], ys[kZonalAhead];
+  // the wave's sum; as a lambda the kernel takes 64 registers and two workgroups of
+  // sixteen waves fit a CU, written out in its place 68 and one (degree 1024, 776
+  // fields: 104 against 117 us)
+  auto partial = [&](int w) {
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int s0 = w; s0 < nsteps; s0 += nw * kZonalAhead) {
+      // steps past the end are not loaded; pairs past P2 load valid addresses and count as 0
+      double a[kZonalAhead], yn[kZonalAhead], ys[kZonalAhead];
 #pragma unroll
-    for (int j = 0; j < kZonalAhead; ++j) {
-      const int s = s0 + j * nw, p = (s < nsteps ? s : 0) * 4 + kq, pc = p < P2 ? p : 0;
-      a[j] = T[(size_t)p * KR];
-      yn[j] = yf[P2 + pc];
-      ys[j] = yf[P2 - 1 - pc];
-    }
+      for (int j = 0; j < kZonalAhead; ++j) {
+        const int s = s0 + j * nw, p = s * 4 + kq, pc = p < P2 ? p : 0;
+        if (s >= nsteps) break;
+        a[j] = T[(size_t)p * KR];
+        yn[j] = yf[P2 + pc];
+        ys[j] = yf[P2 - 1 - pc];
+      }
 #pragma unroll
-    for (int j = 0; j < kZonalAhead; ++j) {
-      const int s = s0 + j * nw;
-      const double v = s < nsteps && s * 4 + kq < P2 && f < nf ? yn[j] + sgn * ys[j] : 0.0;
-      if (s < nsteps) acc = mfma16x4(a[j], v, acc);
+      for (int j = 0; j < kZonalAhead; ++j) {
+        const int s = s0 + j * nw;
+        if (s >= nsteps) break;
+        const double v = s * 4 + kq < P2 && f < nf ? yn[j] + sgn * ys[j] : 0.0;
+        acc = mfma16x4(a[j], v, acc);
+      }
     }
-  }
-  zonal_put(red, wave, lane, acc);
+    return acc;
+  };
+  zonal_put(red, wave, lane, partial(wave));
   __syncthreads();
   const int kn = q ? (N + 1) >> 1 : (N + 2) >> 1;  // degrees of this parity
   for (int e = threadIdx.x; e < 256; e += blockDim.x) {
@@ -134,28 +145,32 @@ __global__ __launch_bounds__(64 * kZonalMaxWaves) void zonal_inv_kernel(
   extern __shared__ double red[];  // [nw][4][64], even halves first
   const int b = blockIdx.x, rt = b % nrt, ct = b / nrt;
   const int wave = wave_id(), nh = blockDim.x >> 7, lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
-  const int q = wave >= nh ? 1 : 0, w = wave - q * nh;
   const int f = ct * 16 + r16;
   const double *__restrict__ lf = l + (size_t)(f < nf ? f : 0) * (N + 1);
-  const double *__restrict__ T = Tinv + (size_t)q * KP * P2p + rt * 16 + r16;
   const int nsteps = KP >> 2;
-  d4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int s0 = w; s0 < nsteps; s0 += nh * kZonalAhead) {
-    double a[kZonalAhead], v[kZonalAhead];
+  auto partial = [&](int q, int w) {
+    const double *__restrict__ T = Tinv + (size_t)q * KP * P2p + rt * 16 + r16;
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int s0 = w; s0 < nsteps; s0 += nh * kZonalAhead) {
+      double a[kZonalAhead], v[kZonalAhead];
 #pragma unroll
-    for (int j = 0; j < kZonalAhead; ++j) {
-      const int s = s0 + j * nh, k = (s < nsteps ? s : 0) * 4 + kq, n = 2 * k + q;
-      a[j] = T[(size_t)k * P2p];
-      v[j] = lf[n <= N ? n : 0];
-    }
+      for (int j = 0; j < kZonalAhead; ++j) {
+        const int s = s0 + j * nh, k = s * 4 + kq, n = 2 * k + q;
+        if (s >= nsteps) break;
+        a[j] = T[(size_t)k * P2p];
+        v[j] = lf[n <= N ? n : 0];
+      }
 #pragma unroll
-    for (int j = 0; j < kZonalAhead; ++j) {
-      const int s = s0 + j * nh;
-      const double x = s < nsteps && 2 * (s * 4 + kq) + q <= N && f < nf ? v[j] : 0.0;
-      if (s < nsteps) acc = mfma16x4(a[j], x, acc);
+      for (int j = 0; j < kZonalAhead; ++j) {
+        const int s = s0 + j * nh;
+        if (s >= nsteps) break;
+        acc = mfma16x4(a[j], 2 * (s * 4 + kq) + q <= N && f < nf ? v[j] : 0.0, acc);
+      }
     }
-  }
-  zonal_put(red, wave, lane, acc);
+    return acc;
+  };
+  const int q = wave >= nh ? 1 : 0;
+  zonal_put(red, wave, lane, partial(q, wave - q * nh));
   __syncthreads();
   for (int e = threadIdx.x; e < 256; e += blockDim.x) {
     const int p = rt * 16 + (e >> 6) * 4 + ((e & 63) >> 4), fo = ct * 16 + (e & 15);
