@@ -66,8 +66,9 @@ static void batch_release(sht_batch *b) {
 }
 
 // The independent pieces of a batch's work: all groups that can share their
-// stages' launches (multi_available) as one piece of up to kMaxMulti groups,
-// largest first, and every other group on its own.  Shared launches because
+// stages' launches (multi_available) as one piece of up to kMaxMulti groups and
+// kMaxMultiBlocks workgroups, largest first, and every other group on its own.
+// Shared launches because
 // small groups' kernels neither fill the chip nor overlap: one after the
 // other each pays its launch and its latency chain, and as branches of a graph
 // they pay the hand-offs between queues.  12 members, T21/T42/T85, fp16, round
@@ -84,8 +85,16 @@ static std::vector<std::vector<int>> batch_units(const sht_batch *b) {
   }
   auto points = [&](int i) { return (size_t)b->groups[i].nf * b->groups[i].jm * b->groups[i].im; };
   std::stable_sort(shared.begin(), shared.end(), [&](int x, int y) { return points(x) > points(y); });
-  for (size_t i = 0; i < shared.size(); i += kMaxMulti)
-    units.emplace_back(shared.begin() + i, shared.begin() + std::min(shared.size(), i + kMaxMulti));
+  long blocks = 0;
+  for (int i : shared) {
+    const long more = multi_blocks(b->groups[i].plan->p, b->groups[i].nf);
+    if (blocks == 0 || blocks + more > kMaxMultiBlocks || units.back().size() == kMaxMulti) {
+      units.emplace_back();
+      blocks = 0;
+    }
+    units.back().push_back(i);
+    blocks += more;
+  }
   return units;
 }
 

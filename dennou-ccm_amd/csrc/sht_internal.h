@@ -334,6 +334,10 @@ struct MultiGroup {
   int nf;
 };
 bool multi_available(const Plan &p, int nf);
+// Workgroups (of 256 threads) of the group's largest stage in such a launch, and
+// the most that a launch may have: the runtime takes less than 2^32 threads.
+long multi_blocks(const Plan &p, int nf);
+constexpr long kMaxMultiBlocks = UINT32_MAX / 256;
 int launch_leg_inv_f64_multi(const MultiGroup *g, int n, hipStream_t s);
 int launch_leg_fwd_f64_multi(const MultiGroup *g, int n, hipStream_t s);
 int launch_leg_inv_mixed_multi(const MultiGroup *g, int n, hipStream_t s);

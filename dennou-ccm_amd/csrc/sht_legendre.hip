@@ -1375,6 +1375,13 @@ bool multi_available(const Plan &p, int nf) {
   return same(resolve_shape(p, nf, 0)) && same(resolve_shape(p, nf, 1));
 }
 
+long multi_blocks(const Plan &p, int nf) {
+  const long nct = (2L * nf + 15) / 16, gf = fft_group(p.im);
+  const long leg = 8L * std::max(p.xcd_mlen[0], p.xcd_mlen[1]) * nct;
+  const long fft = (long)p.P2 * multi_geom(p, nf).nfg * (layout_group(gf) / gf);
+  return (std::max(leg, fft) + 7) / 8 * 8;
+}
+
 int launch_leg_inv_f64(const Plan &p, const double *spec, double *four, double *four2,
                        bool value_table, bool deriv_table, int nf, hipStream_t s) {
   return launch_leg_inv_f64_shape(p, resolve_shape(p, nf, 0), spec, four, four2, value_table,

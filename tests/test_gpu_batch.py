@@ -153,3 +153,26 @@ def test_batch_shared_launches_bitwise(prec, count):
             assert np.array_equal(hipmem.get_member_spectra(spec_out, ld, p.K, nf), shtamd.real_to_spec(so.cpu().numpy())), j
             p.close()
     b.close()
+
+
+def test_batch_groups_beyond_one_launch():
+    """Groups that fill a launch each (2^32 threads) do not share one: degree 0,
+    every grid value is the field's coefficient, and it comes back."""
+    nf = 9 << 20
+    members = [(0, 16, 2, nf), (0, 16, 4, nf)]
+    b = shtamd.Batch(members)
+    rng = np.random.default_rng(3)
+    vals = [rng.standard_normal(nf) for _ in members]
+    for j, v in enumerate(vals):
+        spec_in, _, _, ld = b.member_ptrs(j)
+        hipmem.put_member_spectra(spec_in, ld, v[None, :].astype(complex))
+    b.run(shtamd.DIR_ROUNDTRIP)
+    torch.cuda.synchronize()
+    for j, (_, im, jm, _) in enumerate(members):
+        _, grid, spec_out, ld = b.member_ptrs(j)
+        back = hipmem.get_member_spectra(spec_out, ld, 1, nf)[0]
+        assert np.abs(back - vals[j]).max() < 1e-14, j
+        for f0 in (0, nf // 2 - 500, nf - 1000):
+            g = hipmem.from_device(grid + 8 * f0 * jm * im, (1000, jm * im))
+            assert np.abs(g - vals[j][f0:f0 + 1000, None]).max() < 1e-14, (j, f0)
+    b.close()
