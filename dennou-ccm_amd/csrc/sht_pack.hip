@@ -12,13 +12,65 @@ namespace {
 
 constexpr double kSqrt2 = 1.41421356237309504880;
 
+// Small calls: one thread per (canonical k, field), field fastest: canonical writes coalesce
+__global__ void spml_to_canon_each_kernel(const double *__restrict__ wa, double *__restrict__ spec,
+                                     int N, int nf) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int K = (N + 1) * (N + 2) / 2;
+  if (t >= (int64_t)K * nf) return;
+  const int f = (int)(t % nf);
+  const int k = (int)(t / nf);
+  // invert k = off(m) + n - m: off(m) = m (2N + 3 - m) / 2, so the largest m
+  // with off(m) <= k is the floor of the smaller root of m^2 - (2N+3) m + 2k,
+  // corrected by a step where the square root rounds across an integer
+  const double b = 2.0 * N + 3.0;
+  int m = (int)floor(0.5 * (b - sqrt(b * b - 8.0 * (double)k)));
+  m = m < 0 ? 0 : m > N ? N : m;
+  while (m > 0 && coef_off(N, m) > k) --m;
+  while (m < N && coef_off(N, m + 1) <= k) ++m;
+  const int n = m + (k - (int)coef_off(N, m));
+  const double *w = wa + (size_t)f * (N + 1) * (N + 1);
+  double re, im;
+  if (m == 0) {
+    re = w[n * (n + 1)];
+    im = 0.0;
+  } else {
+    re = w[n * (n + 1) + m] / kSqrt2;
+    im = -w[n * (n + 1) - m] / kSqrt2;
+  }
+  spec[2 * t] = re;
+  spec[2 * t + 1] = im;
+}
+
+// Small calls: one thread per (field, l), l fastest: SPML-layout writes coalesce
+__global__ void canon_to_spml_each_kernel(const double *__restrict__ spec, double *__restrict__ wa,
+                                     int N, int nf) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int L = (N + 1) * (N + 1);
+  if (t >= (int64_t)L * nf) return;
+  const int l = (int)(t % L);
+  const int f = (int)(t / L);
+  int n = (int)sqrt((double)l);
+  while (n * n > l) --n;
+  while ((n + 1) * (n + 1) <= l) ++n;
+  const int m = l - n * (n + 1);
+  const int am = m < 0 ? -m : m;
+  const double *s = spec + ((size_t)(coef_off(N, am) + n - am) * nf + f) * 2;
+  double v;
+  if (m == 0) v = s[0];
+  else if (m > 0) v = kSqrt2 * s[0];
+  else v = -kSqrt2 * s[1];
+  wa[t] = v;
+}
+
 // SPML packing <-> canonical spectra: a workgroup transposes the degree n of
 // kPackFields fields through LDS.  On the SPML side a field's degree is one
 // run of 2n + 1 reals (l = n(n+1) + m, m = -n..n); on the canonical side each
 // (m, n) row holds the fields' complex values next to each other, 128 bytes of
-// them per group.  A thread per element of one side had to gather or scatter
-// single values on the other.  T85, 97 fields (5.7 + 5.8 MB), back to back:
-// to canonical 7.6 -> 5.0 us, to SPML 8.5 -> 4.3 us.
+// them per group.  A thread per element of one side has to gather or scatter
+// single values on the other (the kernels above, for small calls: pack_each).
+// T85, 97 fields (5.7 + 5.8 MB), back to back: to canonical 7.8 -> 4.4 us, to
+// SPML 9.8 -> 4.0 us.
 // The groups of one degree run on one XCD, so the parts of the lines that
 // neighbouring groups share meet in its L2; degrees are dealt to the XCDs in
 // turn, longest first.
@@ -228,6 +280,21 @@ __global__ __launch_bounds__(256) void lapla_kernel(const double2 *in, double2 *
   out[t] = make_double2(x * v.x, x * v.y);
 }
 
+// Which kernel converts a call: one thread per value, or the tiles.  The tiles
+// pay where there are values enough to be bound by lines touched; a tile of few
+// fields leaves most of its lanes idle, one of a short degree (below 32) too, and
+// degrees above 63 take several rounds of rows in few workgroups.  Back to back,
+// per value / tiles, us: to canonical T85 1 field 2.27 / 3.26, 16 fields 2.72 / 2.83,
+// 32 fields 3.23 / 2.99; T42 8 fields equal, 64 fields 2.75 / 2.58; T170 5 fields 2.89 /
+// 3.51, 12 fields 3.80 / 3.63; T21 776 fields 3.91 / 4.87, 1500 fields equal; to SPML
+// T85 1 field 2.05 / 2.42, 16 fields 2.52 / 2.71, 32 fields 3.00 / 2.85; T42 26 fields
+// 2.20 / 2.36, 79 fields 2.55 / 2.52.
+inline bool pack_each(const Plan &p, int nf, bool to_canon) {
+  const int64_t values = (int64_t)p.K * nf;
+  if (p.N < 32 || nf < kPackFields) return values <= 200000;
+  return values <= 65536 && (p.N >= 64 || !to_canon);
+}
+
 }  // namespace
 
 int launch_spec_lapla(const Plan &p, const double *in, double *out, int power, int nf,
@@ -240,17 +307,26 @@ int launch_spec_lapla(const Plan &p, const double *in, double *out, int power, i
 }
 
 int launch_spml_to_canon(const Plan &p, const double *wa, double *spec, int nf, hipStream_t s) {
-  const unsigned tiles = pack_tiles(p.N, nf);
-  spml_to_canon_kernel<<<pack_blocks(tiles), 256, sizeof(double) * kPackFields * pack_pitch(p.N), s>>>(
-      wa, spec, p.N, nf, tiles);
+  if (pack_each(p, nf, true)) {
+    spml_to_canon_each_kernel<<<(unsigned)(((int64_t)p.K * nf + 255) / 256), 256, 0, s>>>(wa, spec, p.N, nf);
+  } else {
+    const unsigned tiles = pack_tiles(p.N, nf);
+    spml_to_canon_kernel<<<pack_blocks(tiles), 256, sizeof(double) * kPackFields * pack_pitch(p.N), s>>>(
+        wa, spec, p.N, nf, tiles);
+  }
   SHT_HIP(hipGetLastError());
   return SHT_OK;
 }
 
 int launch_canon_to_spml(const Plan &p, const double *spec, double *wa, int nf, hipStream_t s) {
-  const unsigned tiles = pack_tiles(p.N, nf);
-  canon_to_spml_kernel<<<pack_blocks(tiles), 256, sizeof(double) * kPackFields * pack_pitch(p.N), s>>>(
-      spec, wa, p.N, nf, tiles);
+  if (pack_each(p, nf, false)) {
+    canon_to_spml_each_kernel<<<(unsigned)(((int64_t)(p.N + 1) * (p.N + 1) * nf + 255) / 256), 256, 0, s>>>(
+        spec, wa, p.N, nf);
+  } else {
+    const unsigned tiles = pack_tiles(p.N, nf);
+    canon_to_spml_kernel<<<pack_blocks(tiles), 256, sizeof(double) * kPackFields * pack_pitch(p.N), s>>>(
+        spec, wa, p.N, nf, tiles);
+  }
   SHT_HIP(hipGetLastError());
   return SHT_OK;
 }

@@ -45,3 +45,20 @@ def test_pack_and_laplacian(N, im, jm, nf, shift):
         p.spec_lapla(a, a, power, nf)
         assert torch.equal(a, out)
     p.close()
+
+
+@pytest.mark.parametrize("N,im,jm,nf", [(10, 32, 16, 3031), (21, 64, 32, 800), (42, 128, 64, 9), (42, 128, 64, 70), (85, 256, 128, 18), (255, 512, 256, 9)])
+def test_pack_both_sides_of_the_line(N, im, jm, nf):
+    """Calls large enough for the tiles: bitwise what small calls of the same fields give."""
+    rng = np.random.default_rng(N)
+    p = shtamd.Plan(N, im, jm, nf)
+    wa = torch.from_numpy(rng.standard_normal((nf, (N + 1) ** 2))).cuda()
+    spec, back = torch.full((p.K, nf, 2), np.nan, dtype=torch.float64, device="cuda"), torch.full_like(wa, np.nan)
+    p.spml_to_canon(wa, spec, nf)
+    p.canon_to_spml(spec, back, nf)
+    for f in (0, 7, nf - 1):
+        s1, w1 = torch.full((p.K, 1, 2), np.nan, dtype=torch.float64, device="cuda"), torch.full_like(wa[:1], np.nan)
+        p.spml_to_canon(wa[f:f + 1].clone(), s1, 1)
+        p.canon_to_spml(s1, w1, 1)
+        assert torch.equal(spec[:, f:f + 1], s1) and torch.equal(back[f:f + 1], w1), f
+    p.close()
