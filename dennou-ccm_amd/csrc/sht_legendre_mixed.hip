@@ -1350,9 +1350,12 @@ int inv_nsl(const Plan &p, int shape, const double *spec, float *four, int nf, h
   }
   if (shape == SHT_SHAPE_STAGED) {
     if (!mixed_stream_available(p)) return fail(SHT_ERR_UNSUPPORTED, "mixed inverse: streaming shape needs <= 128 latitude pairs");
-    // each half of the waves loads two of its tiles (every second one) ahead
+    // each half of the waves loads two of its tiles (every second one) ahead,
+    // one where the table of the six-product form takes the registers (N > 191; N =
+    // 230, two / one: 1 field 12.3 / 8.4 us, 97 fields 38.8 / 29.6, 27 values spilled with two)
+    constexpr int PD = Form<MODE>::NP == 3 && NSL > 3 ? 1 : 2;
     const int cs = stream_chunk(nct);
-    launch_kernel(geo.stream ? leg_inv_mixed_stream_kernel<MODE, NSL, true, 2> : leg_inv_mixed_stream_kernel<MODE, NSL, false, 2>,
+    launch_kernel(geo.stream ? leg_inv_mixed_stream_kernel<MODE, NSL, true, PD> : leg_inv_mixed_stream_kernel<MODE, NSL, false, PD>,
                   xcd_m_blocks(p, 0, (nct + cs - 1) / cs), 1024, 0, s, spec, four,
                   static_cast<const uint16_t *>(p.Linv), p.loff_inv, p.lexp_inv, p.xcd_m[0],
                   p.xcd_mlen[0], p.N, p.P2, p.P2p, ncol, nct, cs, geo);
