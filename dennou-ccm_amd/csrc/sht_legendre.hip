@@ -1270,9 +1270,17 @@ int resolve_shape(const Plan &p, int nf, int dir) {
   }
   // measured on MI355X from T21 to T170 and 16 to 388 fields: the staged
   // shape wins the forward nearly everywhere and the inverse from 32 fields;
-  // below that a wavefront per tile fills the chip better.  STAGED and WAVE
-  // run the same MFMA sequence per output tile, so the switch with the field
-  // count changes no result.
+  // below that a wavefront per tile fills the chip better.  STAGED, WAVE and TILE
+  // run the same MFMA sequence per output tile, so the switches with the field
+  // count change no result.
+  // On at most 32 latitudes (up to 64 with more fields) a staged workgroup's
+  // few K steps are mostly its staging, and TILE runs many fields faster, with the
+  // same sequence again: STAGED / TILE, inverse, forward and both tables, us:
+  // T21 (32 latitudes) 256 fields equal, equal, 5.6 / 4.8; 776 fields 6.2 / 5.6, 5.8 / 4.3,
+  // 9.7 / 9.6; T10 (16 latitudes) 3000 fields 10.5 / 5.5, 11.3 / 5.4, 12.9 / 9.1; N = 31, 64
+  // latitudes 388 fields 7.3 / 7.8, 5.5 / 5.3, 13.5 / 14.4; 776 fields 14.5 / 14.2, 8.9 / 7.5,
+  // 18.3 / 16.2.
+  if (p.P2p <= 32 && nf >= (p.P2p == 16 ? 256 : 512)) return SHT_SHAPE_TILE;
   if (dir == 1) return SHT_SHAPE_STAGED;
   return nf >= 32 ? SHT_SHAPE_STAGED : SHT_SHAPE_WAVE;
 }

@@ -393,3 +393,19 @@ def test_staged_gradients_both_tables_bitwise(N, im, jm, nf):
         got.append(run_inverse(p, spec, nf, grad=True))
     assert all(np.array_equal(a, b) for a, b in zip(*got))
     p.close()
+
+
+@pytest.mark.parametrize("N,im,jm,nf", [(21, 64, 32, 255), (21, 64, 32, 256), (10, 32, 16, 301), (5, 16, 8, 1000), (20, 64, 40, 511), (31, 64, 64, 512)])
+def test_small_grids_built_in_shapes_bitwise(N, im, jm, nf):
+    """The built-in FP64 shapes of grids of up to 64 latitudes around the field counts
+    where they change: values, gradients and the forward are bitwise WAVE's."""
+    spec = synth.spectra(N, nf, cfg=13)
+    p = shtamd.Plan(N, im, jm, nf, flags=shtamd.FLAG_GRAD)
+    assert p.get_shapes(nf) == ((shtamd.SHAPE_STAGED,) * 2 if nf in (255, 511) else (shtamd.SHAPE_TILE,) * 2)
+    grid = np.random.default_rng(N).standard_normal((nf, jm, im))
+    got = []
+    for shape in (shtamd.SHAPE_AUTO, shtamd.SHAPE_WAVE):
+        p.set_shapes(nf, shape, shape)
+        got.append(run_inverse(p, spec, nf) + run_inverse(p, spec, nf, grad=True) + [run_forward(p, grid, nf)])
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    p.close()
