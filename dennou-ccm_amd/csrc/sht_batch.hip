@@ -66,13 +66,18 @@ static void batch_release(sht_batch *b) {
 }
 
 // The independent pieces of a batch's work: all groups that can share their
-// stages' launches (multi_available) as one piece of up to kMaxMulti groups and
-// kMaxMultiBlocks workgroups, largest first, and every other group on its own.
-// Shared launches because
+// stages' launches (multi_available) as one piece of up to kMaxMulti groups,
+// kMaxMultiBlocks workgroups and kMaxMultiGrid bytes of grids, largest first, and
+// every other group on its own.  Shared launches because
 // small groups' kernels neither fill the chip nor overlap: one after the
 // other each pays its launch and its latency chain, and as branches of a graph
 // they pay the hand-offs between queues.  12 members, T21/T42/T85, fp16, round
-// trip: 84.5 us group by group, 89-110 us as graph branches, 55 us shared.
+// trip: 84.5 us group by group, 89-110 us as graph branches, 55 us shared.  Large
+// groups lose by it: a group's stages then no longer follow each other while its
+// data are in the Infinity Cache.  T42 and T85 of 800 / 1200 / 1500 fields each (262 /
+// 393 / 491 MB of grids), FP64, shared 228 / 399 / 568 us, graph branches 226 / 388 /
+// 523; x6 205 / 293 / 402 and 205 / 284 / 397; T21 and T42 of 5000 (410 MB), x6 333 and 292.
+constexpr size_t kMaxMultiGrid = 400000000;
 static std::vector<std::vector<int>> batch_units(const sht_batch *b) {
   std::vector<int> shared;
   std::vector<std::vector<int>> units;
@@ -83,17 +88,23 @@ static std::vector<std::vector<int>> batch_units(const sht_batch *b) {
     else
       units.push_back({i});
   }
-  auto points = [&](int i) { return (size_t)b->groups[i].nf * b->groups[i].jm * b->groups[i].im; };
-  std::stable_sort(shared.begin(), shared.end(), [&](int x, int y) { return points(x) > points(y); });
+  auto grid_bytes = [&](int i) {
+    return sizeof(double) * b->groups[i].nf * b->groups[i].jm * b->groups[i].im;
+  };
+  std::stable_sort(shared.begin(), shared.end(), [&](int x, int y) { return grid_bytes(x) > grid_bytes(y); });
   long blocks = 0;
+  size_t bytes = 0;
   for (int i : shared) {
     const long more = multi_blocks(b->groups[i].plan->p, b->groups[i].nf);
-    if (blocks == 0 || blocks + more > kMaxMultiBlocks || units.back().size() == kMaxMulti) {
+    if (blocks == 0 || blocks + more > kMaxMultiBlocks || bytes + grid_bytes(i) > kMaxMultiGrid ||
+        units.back().size() == kMaxMulti) {
       units.emplace_back();
       blocks = 0;
+      bytes = 0;
     }
     units.back().push_back(i);
     blocks += more;
+    bytes += grid_bytes(i);
   }
   return units;
 }
