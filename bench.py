@@ -534,7 +534,8 @@ def run_ensemble(precision: str, nmember: int, steps: int, warmup: int, seed: in
         spec_in, _, _, ld = b.member_ptrs(j)
         hipmem.put_member_spectra(spec_in, ld, s)
         specs.append(s)
-    # per-group Legendre shapes from the autotuner, then the graph is captured
+    # per-group Legendre shapes, and whether the smaller groups share their
+    # launches, from the autotuner; then the graph is captured
     b.autotune(reps=5, shapes_only=shapes_only)
     stream = torch.cuda.current_stream()
     for _ in range(max(1, warmup)):

@@ -22,6 +22,7 @@ namespace sht {
 
 struct BatchGroup {
   int nmax = 0, im = 0, jm = 0, nf = 0;
+  bool can_share = false;  // its built-in shapes' results are those of the shared launches
   sht_plan *plan = nullptr;
   double *spec_in = nullptr, *grid = nullptr, *spec_out = nullptr;
   hipStream_t stream = nullptr;
@@ -41,6 +42,7 @@ struct sht_batch {
   std::vector<sht::BatchGroup> groups;
   std::vector<sht::BatchMember> members;
   std::vector<std::vector<int>> units;  // group indexes, see batch_units
+  bool share = true;                    // see pick_sharing
   hipEvent_t fork = nullptr;
   hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
   hipGraph_t graph[3] = {nullptr, nullptr, nullptr};
@@ -48,11 +50,17 @@ struct sht_batch {
 
 namespace sht {
 
-static void batch_release(sht_batch *b) {
+static void drop_graphs(sht_batch *b) {
   for (int d = 0; d < 3; ++d) {
     if (b->exec[d]) (void)hipGraphExecDestroy(b->exec[d]);
     if (b->graph[d]) (void)hipGraphDestroy(b->graph[d]);
+    b->exec[d] = nullptr;
+    b->graph[d] = nullptr;
   }
+}
+
+static void batch_release(sht_batch *b) {
+  drop_graphs(b);
   for (auto &g : b->groups) {
     if (g.plan) sht_plan_destroy(g.plan);
     if (g.spec_in) (void)hipFree(g.spec_in);
@@ -82,8 +90,7 @@ static std::vector<std::vector<int>> batch_units(const sht_batch *b) {
   std::vector<int> shared;
   std::vector<std::vector<int>> units;
   for (int i = 0; i < (int)b->groups.size(); ++i) {
-    const BatchGroup &g = b->groups[i];
-    if (multi_available(g.plan->p, g.nf))
+    if (b->share && b->groups[i].can_share)
       shared.push_back(i);
     else
       units.push_back({i});
@@ -149,6 +156,104 @@ static int enqueue_all(sht_batch *b, int dir, hipStream_t s, bool fork_join) {
     }
   }
   return SHT_OK;
+}
+
+// All units of one direction on s: directly if there is one, else as a graph,
+// captured on the first call.
+static int run_units(sht_batch *b, int dir, hipStream_t s) {
+  // a single piece has no branches to run side by side, and its launches take
+  // less than a graph's
+  if (b->units.size() == 1) return enqueue_all(b, dir, s, false);
+  if (!b->exec[dir]) {
+    // capture on a private stream so the caller's stream may be the legacy one
+    hipStream_t cap = nullptr;
+    SHT_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
+    hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
+    int rc = (e == hipSuccess) ? enqueue_all(b, dir, cap, true)
+                               : fail(SHT_ERR_DEVICE, "sht_batch_run: hipStreamBeginCapture failed");
+    hipGraph_t graph = nullptr;
+    hipError_t e2 = hipStreamEndCapture(cap, &graph);
+    (void)hipStreamDestroy(cap);
+    if (rc) {
+      if (graph) (void)hipGraphDestroy(graph);
+      return rc;
+    }
+    if (e2 != hipSuccess) return fail(SHT_ERR_DEVICE, "sht_batch_run: hipStreamEndCapture failed");
+    hipGraphExec_t exec = nullptr;
+    if (hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) {
+      (void)hipGraphDestroy(graph);
+      return fail(SHT_ERR_DEVICE, "sht_batch_run: hipGraphInstantiate failed");
+    }
+    b->graph[dir] = graph;
+    b->exec[dir] = exec;
+  }
+  SHT_HIP(hipGraphLaunch(b->exec[dir], s));
+  return SHT_OK;
+}
+
+// Whether the groups that can share launches are to: times the round trip of
+// those groups' shared launches against that of each group's own kernels (the
+// tuned shapes), on scratch data and the plans' own Fourier scratch, and keeps
+// sharing unless the latter is at least 3 % faster.  Without memory for the
+// scratch data the choice stays.  Called while the batch is idle.
+static int pick_sharing(sht_batch *b, int reps) {
+  sht_batch t;  // the groups in question over scratch data
+  b->share = true;
+  for (const auto &u : batch_units(b))
+    if (u.size() > 1)
+      for (int i : u) t.groups.push_back(b->groups[i]);
+  if (t.groups.empty()) return SHT_OK;
+  t.fork = b->fork;
+  int cur = 0, rc = SHT_OK;
+  bool memory = true;
+  hipStream_t s = nullptr;
+  hipEvent_t e[2] = {nullptr, nullptr};
+  SHT_HIP(hipGetDevice(&cur));
+  SHT_HIP(hipSetDevice(t.groups[0].plan->p.device));
+  for (auto &g : t.groups) g.spec_in = g.spec_out = g.grid = nullptr;
+  for (auto &g : t.groups) {
+    const size_t nspec = sizeof(double) * g.plan->p.K * 2 * g.nf, ngrid = sizeof(double) * g.nf * g.jm * g.im;
+    memory = hipMalloc(&g.spec_in, nspec) == hipSuccess && hipMalloc(&g.grid, ngrid) == hipSuccess &&
+             hipMemset(g.spec_in, 0, nspec) == hipSuccess && hipMemset(g.grid, 0, ngrid) == hipSuccess;
+    g.spec_out = g.spec_in;
+    if (!memory) break;
+  }
+  double best[2] = {0.0, 0.0};
+  if (memory) {
+    if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&e[0]) != hipSuccess ||
+        hipEventCreate(&e[1]) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
+      rc = fail(SHT_ERR_DEVICE, "sht_batch_autotune: stream or event creation failed");
+    // three interleaved rounds, as for the shapes: a drift hits both alike
+    for (int round = 0; round < 6 && !rc; ++round) {
+      t.share = round % 2 == 0;
+      t.units = batch_units(&t);
+      drop_graphs(&t);
+      rc = run_units(&t, SHT_DIR_ROUNDTRIP, s);  // captures, loads code
+      if (!rc) rc = run_units(&t, SHT_DIR_ROUNDTRIP, s);
+      if (!rc && hipEventRecord(e[0], s) != hipSuccess) rc = fail(SHT_ERR_DEVICE, "sht_batch_autotune: hipEventRecord");
+      for (int r = 0; r < reps && !rc; ++r) rc = run_units(&t, SHT_DIR_ROUNDTRIP, s);
+      float ms = 0.f;
+      if (!rc && (hipEventRecord(e[1], s) != hipSuccess || hipEventSynchronize(e[1]) != hipSuccess ||
+                  hipEventElapsedTime(&ms, e[0], e[1]) != hipSuccess))
+        rc = fail(SHT_ERR_DEVICE, "sht_batch_autotune: timing failed");
+      double &x = best[t.share ? 0 : 1];
+      if (!rc && (round < 2 || ms < x)) x = ms;
+    }
+    (void)hipDeviceSynchronize();
+    b->share = rc || best[1] > 0.97 * best[0];
+  } else {
+    (void)hipGetLastError();
+  }
+  drop_graphs(&t);
+  for (auto &g : t.groups) {
+    if (g.spec_in) (void)hipFree(g.spec_in);
+    if (g.grid) (void)hipFree(g.grid);
+  }
+  for (hipEvent_t x : e)
+    if (x) (void)hipEventDestroy(x);
+  if (s) (void)hipStreamDestroy(s);
+  (void)hipSetDevice(cur);
+  return rc;
 }
 
 }  // namespace sht
@@ -229,6 +334,7 @@ int sht_batch_create(const sht_member_desc *members, int nmember, int precision,
     batch_release(b);
     return fail(SHT_ERR_DEVICE, "sht_batch_create: device synchronisation failed");
   }
+  for (auto &g : b->groups) g.can_share = multi_available(g.plan->p, g.nf);
   b->units = batch_units(b);
   *out = b;
   return SHT_OK;
@@ -255,35 +361,7 @@ int sht_batch_run(sht_batch *b, int dir, void *stream) {
   if (!b) return fail(SHT_ERR_INVALID, "sht_batch_run: batch is NULL");
   if (dir < SHT_DIR_INVERSE || dir > SHT_DIR_ROUNDTRIP)
     return fail(SHT_ERR_INVALID, "sht_batch_run: bad direction");
-  hipStream_t s = (hipStream_t)stream;
-  // a single piece has no branches to run side by side, and its launches take
-  // less than a graph's
-  if (b->units.size() == 1) return enqueue_all(b, dir, s, false);
-  if (!b->exec[dir]) {
-    // capture on a private stream so the caller's stream may be the legacy one
-    hipStream_t cap = nullptr;
-    SHT_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
-    hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
-    int rc = (e == hipSuccess) ? enqueue_all(b, dir, cap, true)
-                               : fail(SHT_ERR_DEVICE, "sht_batch_run: hipStreamBeginCapture failed");
-    hipGraph_t graph = nullptr;
-    hipError_t e2 = hipStreamEndCapture(cap, &graph);
-    (void)hipStreamDestroy(cap);
-    if (rc) {
-      if (graph) (void)hipGraphDestroy(graph);
-      return rc;
-    }
-    if (e2 != hipSuccess) return fail(SHT_ERR_DEVICE, "sht_batch_run: hipStreamEndCapture failed");
-    hipGraphExec_t exec = nullptr;
-    if (hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) {
-      (void)hipGraphDestroy(graph);
-      return fail(SHT_ERR_DEVICE, "sht_batch_run: hipGraphInstantiate failed");
-    }
-    b->graph[dir] = graph;
-    b->exec[dir] = exec;
-  }
-  SHT_HIP(hipGraphLaunch(b->exec[dir], s));
-  return SHT_OK;
+  return run_units(b, dir, (hipStream_t)stream);
 }
 
 int sht_batch_autotune(sht_batch *b, int reps, const char *cache_path) {
@@ -295,18 +373,17 @@ int sht_batch_autotune_flags(sht_batch *b, int reps, const char *cache_path, int
   // the tuner runs on a stream of its own through each group plan's Fourier
   // scratch: a graph or eager run still in flight on any stream would share it
   SHT_HIP(hipDeviceSynchronize());
+  // graphs captured before hold the old kernels (dropped before the first shape
+  // changes, so that an error leaves none): capture again on the next run
+  drop_graphs(b);
+  int rc = SHT_OK;
   for (auto &g : b->groups) {
-    int rc = sht_plan_autotune_flags(g.plan, g.nf, reps, cache_path, flags, nullptr);
-    if (rc) return rc;
+    rc = sht_plan_autotune_flags(g.plan, g.nf, reps, cache_path, flags, nullptr);
+    if (rc) break;
   }
+  if (!rc) rc = pick_sharing(b, reps);
   b->units = batch_units(b);
-  // graphs captured before hold the old kernels: capture again on the next run
-  for (int d = 0; d < 3; ++d) {
-    if (b->exec[d]) (void)hipGraphExecDestroy(b->exec[d]);
-    if (b->graph[d]) (void)hipGraphDestroy(b->graph[d]);
-    b->exec[d] = nullptr;
-    b->graph[d] = nullptr;
-  }
+  if (rc) return rc;
   SHT_HIP(hipDeviceSynchronize());
   return SHT_OK;
 }

@@ -560,8 +560,9 @@ class Batch:
 
     def autotune(self, reps: int = 10, cache_path: str | None = None, shapes_only: bool = False):
         """Tune every group's Legendre shapes (and, for FP64 groups unless
-        shapes_only, the split shape's wavenumber classes) at its field count;
-        recapture on the next run."""
+        shapes_only, the split shape's wavenumber classes) at its field count
+        and whether the groups that can share launches do; recapture on the
+        next run."""
         check(lib().sht_batch_autotune_flags(self._h, reps, cache_path.encode() if cache_path else None,
                                              TUNE_SHAPES_ONLY if shapes_only else 0))
 

@@ -220,8 +220,9 @@ int sht_restart_read(const char *path, const sht_restart_desc *desc, double *tim
  *      ensemble runs.  Members are grouped by grid (nmax, im, jm); each group's
  *      members are consecutive field ranges of one resident batch, so every
  *      kernel launch covers all members of a group; groups of at most 64
- *      latitude pairs and 256 longitudes share one launch per stage, and
- *      larger ones run beside them as branches of a hipGraph.                */
+ *      latitude pairs and 256 longitudes share one launch per stage (up to
+ *      400 MB of grids together), and larger ones run beside them as branches
+ *      of a hipGraph.                                                        */
 typedef struct sht_batch sht_batch;
 typedef struct {
   int nmax, im, jm; /* truncation and grid of the member */
@@ -247,9 +248,13 @@ int sht_batch_run(sht_batch *batch, int direction, void *stream);
 /* The same work launched kernel by kernel (no graph), for comparison. */
 int sht_batch_run_eager(sht_batch *batch, int direction, void *stream);
 /* Autotunes the Legendre kernel shapes of every group's plan at the group's
- * field count (sht_plan_autotune; cache_path may be NULL), then drops the
- * captured graphs so the next sht_batch_run captures the tuned kernels.
- * Synchronizes the device; call it while the batch is idle. */
+ * field count (sht_plan_autotune; cache_path may be NULL), then, if groups share
+ * launches (sht_batch_create), times those against the same groups each with its
+ * own tuned kernels and keeps the faster: groups that go on sharing run the
+ * shared launches' kernels whatever shape was tuned for them alone.  Captured
+ * graphs are dropped, so the next sht_batch_run captures the choice.  The
+ * members' buffers keep their contents.  Synchronizes the device; call it while
+ * the batch is idle. */
 int sht_batch_autotune(sht_batch *batch, int reps, const char *cache_path);
 /* The same with sht_plan_autotune_flags' flags. */
 int sht_batch_autotune_flags(sht_batch *batch, int reps, const char *cache_path, int flags);

@@ -176,3 +176,78 @@ def test_batch_groups_beyond_one_launch():
             g = hipmem.from_device(grid + 8 * f0 * jm * im, (1000, jm * im))
             assert np.abs(g - vals[j][f0:f0 + 1000, None]).max() < 1e-14, (j, f0)
     b.close()
+
+
+BIG = (100, 256, 202)  # more latitude pairs than a shared launch takes: a branch of its own
+
+
+def round_trip_us(b, n=20):
+    b.run(shtamd.DIR_ROUNDTRIP)
+    best = float("inf")
+    for _ in range(5):
+        t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        torch.cuda.synchronize()
+        t0.record()
+        for _ in range(n):
+            b.run(shtamd.DIR_ROUNDTRIP)
+        t1.record()
+        torch.cuda.synchronize()
+        best = min(best, t0.elapsed_time(t1) / n * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("prec", [shtamd.PREC_FP64, shtamd.PREC_SPLIT_BF16X6])
+def test_batch_captured_graph_replays_and_is_dropped(prec):
+    """A batch of shared and single groups runs as a graph: replays equal the eager run,
+    and tuning after a capture keeps the members' data and gives a new graph that
+    equals the eager run again."""
+    members = [(21, 64, 32, 9), (42, 128, 64, 5), (*BIG, 6)]
+    b = shtamd.Batch(members, precision=prec)
+    specs = [synth.spectra(m[0], m[3], cfg=6, member=j) for j, m in enumerate(members)]
+
+    def read():
+        torch.cuda.synchronize()
+        out = []
+        for j, (N, im, jm, nf) in enumerate(members):
+            _, grid, spec_out, ld = b.member_ptrs(j)
+            out += [hipmem.from_device(grid, (nf, jm, im)), hipmem.get_member_spectra(spec_out, ld, shtamd.ncoef(N), nf)]
+        return out
+
+    def fill(which, value):
+        for j, (N, im, jm, nf) in enumerate(members):
+            spec_in, _, spec_out, ld = b.member_ptrs(j)
+            hipmem.put_member_spectra(spec_in if which == "in" else spec_out, ld, specs[j] if value is None else np.full((shtamd.ncoef(N), nf), value, dtype=complex))
+
+    scratch = torch.zeros(1 << 20, dtype=torch.float64, device="cuda")
+    fill("in", None)
+    for tuned in (False, True):
+        b.run_eager(shtamd.DIR_ROUNDTRIP)
+        ref = read()
+        for rep in range(3):
+            scratch.add_(1.0)
+            fill("out", 7.0)
+            b.run(shtamd.DIR_ROUNDTRIP)
+            assert all(np.array_equal(x, y) for x, y in zip(read(), ref)), (tuned, rep)
+        if not tuned:
+            b.autotune(reps=2)
+            assert all(np.array_equal(x, y) for x, y in zip(read(), ref))  # buffers untouched
+    for j, (N, im, jm, nf) in enumerate(members):
+        assert np.linalg.norm(ref[2 * j + 1] - specs[j]) / np.linalg.norm(specs[j]) < (1e-12 if prec == shtamd.PREC_FP64 else 2e-6)
+    b.close()
+
+
+@pytest.mark.parametrize("prec", [shtamd.PREC_FP64, shtamd.PREC_SCALED_FP16])
+def test_batch_autotune_keeps_shared_launches(prec, tmp_path):
+    """Groups whose tuned shape (here forced by a cache: K-split) is not the shared
+    launches' stay in these where they are faster, as for small grids by far (20 us
+    against 65 as graph branches): a tuned batch is not slower."""
+    members = [(21, 64, 32, 49), (42, 128, 64, 40)]
+    cache = tmp_path / "shapes.json"
+    cache.write_text("{" + ", ".join(f'"T{N}_{im}x{jm}_nf{nf}_p{prec}": [0, 0, -1, -1, -1, -1]' for N, im, jm, nf in members) + "}")
+    b = shtamd.Batch(members, precision=prec)
+    before = round_trip_us(b)
+    b.autotune(reps=3, cache_path=str(cache))
+    after = round_trip_us(b)
+    print(f"round trip {before:.1f} us, tuned {after:.1f} us", flush=True)
+    assert after < 1.4 * before
+    b.close()
