@@ -968,10 +968,10 @@ int inv_staged_launch(const Plan &p, const double *spec, double *four, double *f
   // 23.8 / 22.0; T170 64 fields 40.8 / 44.9, 192 fields 111 / 107.
   const int nwg = xcd_m_blocks(p, 0, (nct + CT - 1) / CT);
   const bool merge = ntab == 2 && nwg >= (p.P2p / 8 <= NW ? 1024 : 2048);
-  launch_kernel(merge ? (geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true, true>
-                                    : leg_inv_f64_staged_kernel<CT, 4, NW, false, true>)
-                      : (geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true, false>
-                                    : leg_inv_f64_staged_kernel<CT, 4, NW, false, false>),
+  auto kern = geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true, false> : leg_inv_f64_staged_kernel<CT, 4, NW, false, false>;
+  if constexpr (CT > 1 || NW < 8)  // one tile and eight waves: one table only (kOneTileMaxFields)
+    if (merge) kern = geo.stream ? leg_inv_f64_staged_kernel<CT, 4, NW, true, true> : leg_inv_f64_staged_kernel<CT, 4, NW, false, true>;
+  launch_kernel(kern,
       merge ? nwg : xcd_m_blocks(p, 0, ntab * ((nct + CT - 1) / CT)), NW * 64, inv_staged_lds(p, CT), s, spec, four, four2, p.Pinv, p.Hinv,
       p.poff_inv, p.xcd_m[0], p.xcd_mlen[0], p.N, p.P2, p.P2p, ncol, nct, tab0, ntab, geo);
   SHT_HIP(hipGetLastError());

@@ -334,8 +334,8 @@ __device__ __forceinline__ void put_four4(float *dst, f4 v) {
 template <int MODE, int NSL, bool NT, bool COH>
 __device__ __forceinline__ void inv_tile(const uint16_t *bt, const int *ebits, float *ob,
                                          const uint4 (&pa)[2][NSL][3], double ea0, double ea1, int nsl,
-                                         float *__restrict__ four, FourGeom geo, int P2, int ncol, int m,
-                                         int rt, int jt, int lane) {
+                                         float *__restrict__ four, FourGeom geo, int P2, int m, int rt, int jt,
+                                         int lane) {
   const int r16 = lane & 15, kq = lane >> 4;
   d4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
 #pragma unroll
@@ -458,8 +458,8 @@ __device__ __forceinline__ void leg_inv_mixed_item(
     for (int j = 0; j < CT; ++j) {
       if (j >= nc) break;
       inv_tile<MODE, NSL, NT, COH>(bt + (size_t)j * NG * NP * 16 * kRowPitch, ebits + j * NG * 16,
-                                   obuf + wave * (16 * kOutPitch), pa, ea0, ea1, nsl, four, geo, P2, ncol,
-                                   m, rt, ct0 + j, lane);
+                                   obuf + wave * (16 * kOutPitch), pa, ea0, ea1, nsl, four, geo, P2, m, rt,
+                                   ct0 + j, lane);
     }
     if constexpr (ONE) break;
   }
@@ -1470,7 +1470,7 @@ int fwd_nsl(const Plan &p, int shape, const float *four, double *spec, int nf, h
     SHT_HIP(hipGetLastError());
     return SHT_OK;
   }
-  if constexpr (NSL <= 4) {
+  if constexpr (NSL == 4) {  // of the 128-pair grids
     if (shape == SHT_SHAPE_TILE && p.P2p == 128 && fwd_streams<MODE>(nf)) {
       const int cs = stream_chunk(nct);
       launch_kernel(leg_fwd_mixed_stream_kernel<MODE, NSL, MODE == SHT_PREC_SPLIT_BF16 ? 2 : 1>, xcd_m_blocks(p, 1, (nct + cs - 1) / cs), 1024, 0, s, four,

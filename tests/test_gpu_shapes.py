@@ -409,3 +409,18 @@ def test_small_grids_built_in_shapes_bitwise(N, im, jm, nf):
         got.append(run_inverse(p, spec, nf) + run_inverse(p, spec, nf, grad=True) + [run_forward(p, grid, nf)])
     assert all(np.array_equal(a, b) for a, b in zip(*got))
     p.close()
+
+
+@pytest.mark.parametrize("N,im,jm,nf", [(42, 128, 64, 168), (42, 128, 64, 169), (85, 256, 128, 184), (85, 256, 128, 185), (170, 512, 256, 176), (170, 512, 256, 177)])
+def test_staged_gradients_across_the_line_bitwise(N, im, jm, nf):
+    """The staged inverse just below the line, a workgroup per table (T42 168 fields:
+    1,008 workgroups of 1,024; T85 184: 2,024 of 2,048; T170 176, two column tiles each:
+    1,936), and just above it, both tables in one: bitwise WAVE."""
+    spec = synth.spectra(N, nf, cfg=14)
+    p = shtamd.Plan(N, im, jm, nf, flags=shtamd.FLAG_GRAD)
+    got = []
+    for shape in (shtamd.SHAPE_WAVE, shtamd.SHAPE_STAGED):
+        p.set_shapes(nf, shape, shtamd.SHAPE_AUTO)
+        got.append(run_inverse(p, spec, nf, grad=True))
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    p.close()
