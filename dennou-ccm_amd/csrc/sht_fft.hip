@@ -289,6 +289,8 @@ template <bool FWD>
 int multi_launch(const MultiGroup *g, int n, hipStream_t s) {
   FftMulti a{};
   a.ng = n;
+  // fft_multi_kernel holds as many blocks per CU as the single kernels whose
+  // residency the plans have: four by their 32 KB of LDS, five by its registers
   int nblk = 0, total = 0, resident = INT32_MAX;
   for (int i = 0; i < n; ++i) {
     const Plan &p = *g[i].p;
