@@ -287,12 +287,12 @@ __global__ __launch_bounds__(256) void lapla_kernel(const double2 *in, double2 *
 // per value / tiles, us: to canonical T85 1 field 2.27 / 3.26, 16 fields 2.72 / 2.83,
 // 32 fields 3.23 / 2.99; T42 8 fields equal, 64 fields 2.75 / 2.58; T170 5 fields 2.89 /
 // 3.51, 12 fields 3.80 / 3.63; T21 776 fields 3.91 / 4.87, 1500 fields equal; to SPML
-// T85 1 field 2.05 / 2.42, 16 fields 2.52 / 2.71, 32 fields 3.00 / 2.85; T42 26 fields
+// T85 1 field 2.05 / 2.42, 24 fields 2.69 / 2.79, 32 fields 3.00 / 2.85; T42 26 fields
 // 2.20 / 2.36, 79 fields 2.55 / 2.52.
 inline bool pack_each(const Plan &p, int nf, bool to_canon) {
   const int64_t values = (int64_t)p.K * nf;
   if (p.N < 32 || nf < kPackFields) return values <= 200000;
-  return values <= 65536 && (p.N >= 64 || !to_canon);
+  return p.N < 64 ? !to_canon && values <= 65536 : values <= (to_canon ? 65536 : 100000);
 }
 
 }  // namespace
