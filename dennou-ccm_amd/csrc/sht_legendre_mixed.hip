@@ -1453,10 +1453,14 @@ int build_fused(Plan &p) {
 // fields 16.4 / 16.0, 145 fields 38.2 / 34.9, 388 fields 81.8 / 65.3, 776 fields
 // 161 / 139; BF16 x3 8 fields 6.4 / 5.9, 33 fields 10.2 / 10.8, 388 fields 69.0 /
 // 55.4, 776 fields 129 / 115; scaled FP16 145 fields 32.7 / 32.8, 388 fields
-// 69.8 / 61.6.
+// 69.8 / 61.6.  The third column tile of each m (17 to 24 fields) pays up to 14 table
+// waves (N <= 223), 10 in the scaled form, whose conversions are longer: 24 fields,
+// x6 N = 200 13.1 / 12.5, N = 255 14.4 / 15.5; BF16 x3 10.1 / 9.6 and 10.8 / 11.8; scaled
+// FP16 N = 140 8.3 / 7.8, 170 8.9 / 9.4, 255 11.0 / 13.2.
 template <int MODE>
-bool fwd_streams(int nf) {
-  return nf <= 24 || nf >= (MODE == SHT_PREC_SPLIT_BF16X6 ? 56 : 192);
+bool fwd_streams(const Plan &p, int nf) {
+  const int few = ceil_half(p.N + 1) <= (Form<MODE>::kScaled ? 80 : 112) ? 24 : 16;
+  return nf <= few || nf >= (MODE == SHT_PREC_SPLIT_BF16X6 ? 56 : 192);
 }
 
 template <int MODE, int NSL>
@@ -1471,7 +1475,7 @@ int fwd_nsl(const Plan &p, int shape, const float *four, double *spec, int nf, h
     return SHT_OK;
   }
   if constexpr (NSL == 4) {  // of the 128-pair grids
-    if (shape == SHT_SHAPE_TILE && p.P2p == 128 && fwd_streams<MODE>(nf)) {
+    if (shape == SHT_SHAPE_TILE && p.P2p == 128 && fwd_streams<MODE>(p, nf)) {
       const int cs = stream_chunk(nct);
       launch_kernel(leg_fwd_mixed_stream_kernel<MODE, NSL, MODE == SHT_PREC_SPLIT_BF16 ? 2 : 1>, xcd_m_blocks(p, 1, (nct + cs - 1) / cs), 1024, 0, s, four,
                     spec, static_cast<const uint16_t *>(p.Lfwd), p.loff_fwd, p.lexp_fwd, p.xcd_m[1], p.xcd_mlen[1],

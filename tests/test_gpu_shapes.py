@@ -424,3 +424,20 @@ def test_staged_gradients_across_the_line_bitwise(N, im, jm, nf):
         got.append(run_inverse(p, spec, nf, grad=True))
     assert all(np.array_equal(a, b) for a, b in zip(*got))
     p.close()
+
+
+@pytest.mark.parametrize("prec", [shtamd.PREC_SPLIT_BF16, shtamd.PREC_SCALED_FP16, shtamd.PREC_SPLIT_BF16X6])
+@pytest.mark.parametrize("N,jm", [(159, 240), (160, 256), (223, 256), (224, 256)])
+def test_mixed_forward_third_tile_bitwise(prec, N, jm):
+    """The forward of three column tiles on 128 pairs, streamed or not by degree and
+    form, and the streaming inverse of the six-product form either side of degree
+    191: bitwise the K-split shape's."""
+    p = shtamd.Plan(N, 512, jm, 24, precision=prec)
+    grid = np.random.default_rng(N).standard_normal((24, jm, 512))
+    spec = synth.spectra(N, 24, cfg=15)
+    got = []
+    for shape in (shtamd.SHAPE_KSPLIT, shtamd.SHAPE_TILE):
+        p.set_shapes(24, shape if shape == shtamd.SHAPE_KSPLIT else shtamd.SHAPE_STAGED, shape)
+        got.append((run_inverse(p, spec, 24)[0], run_forward(p, grid, 24), run_forward(p, grid[:16], 16), run_forward(p, grid[:17], 17)))
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    p.close()
