@@ -226,9 +226,13 @@ __global__ __launch_bounds__(1024) void avr_kernel(const double *__restrict__ gr
   __shared__ double red[16];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int q = 1; q < (int)blockDim.x >> 6; ++q) acc += red[q];
-    avg[f] = acc / (2.0 * im);
+  // the waves' sums pairwise: added in a row, their roundings are half as large
+  // again as all others together (256 x 128, rms error 1.2e-16 against 0.9e-16)
+  if (threadIdx.x < 16) {
+    acc = threadIdx.x < blockDim.x >> 6 ? red[threadIdx.x] : 0.0;
+#pragma unroll
+    for (int s = 8; s > 0; s >>= 1) acc += __shfl_xor(acc, s);
+    if (threadIdx.x == 0) avg[f] = acc / (2.0 * im);
   }
 }
 // a wave for each 64 x 2 kAvrAhead points, up to 16 waves

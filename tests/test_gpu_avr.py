@@ -33,3 +33,22 @@ def test_avr_of_several_rounds(N, im, jm, shift):
     """Fields of one full round and a little more, of a part-filled last round, of
     the most rows: against the oracle, at most 512 x 256 terms as above."""
     test_avr_against_oracle(N, im, jm, shift)
+
+
+@pytest.mark.parametrize("N,im,jm", [(42, 128, 64), (85, 256, 128), (106, 512, 160), (170, 512, 256)])
+def test_avr_rounding_errors(N, im, jm):
+    """The sum is a tree over threads and waves.  One addition rounds by 0.46e-16 rms (a uniform
+    half ulp over the mantissas); a tree's last levels add up to sqrt(1 + 1/2 + 1/4 + ...) of
+    these, the division by 2 im one more: 0.8e-16.  Sixteen waves' sums added in a row have
+    sqrt(2^2 + ... + 16^2) / 16 = 2.4 instead: 1.2e-16."""
+    nf = 400
+    mid = np.linspace(-0.5, 0.5, jm) * np.pi
+    g = 2.0 * np.random.default_rng(1).standard_normal((nf, jm, im)) + (200.0 + 100.0 * np.cos(mid) ** 2)[None, :, None]
+    p = shtamd.Plan(N, im, jm, nf)
+    w = np.asarray(p.grid()[3])
+    avg = torch.empty(nf, dtype=torch.float64, device="cuda")
+    p.avr_lonlat(torch.from_numpy(g).cuda(), avg, nf)
+    ref = (g.astype(np.longdouble).sum(-1) * w.astype(np.longdouble)).sum(-1) / (2 * im)
+    err = ((avg.cpu().numpy() - ref) / ref).astype(float)
+    assert np.sqrt((err * err).mean()) < 1.05e-16
+    p.close()
