@@ -34,7 +34,8 @@ constexpr int kThreadsOf = C / 8;
 // big block, with the twiddles in LDS too 41-45 KB: 3 blocks per CU at 512
 // longitudes, where 32 KB allow 4.  T170 (512 longitudes), inverse / forward:
 // 776 fields FP32 225 / 217 -> 199 / 194 us, 145 fields FP64 54 / 54 -> 46.6 /
-// 47.0; up to 256 longitudes, 4 blocks per CU either way, the times stay.
+// 47.0; up to 256 longitudes, 4 blocks per CU either way, T85 gains 4-7 % and T42
+// loses 1-2 % from 388 fields on (FP64).
 // swz is linear in the bits, so for indexes without common bits swz(a + c) =
 // swz(a) ^ swz(c): a butterfly's accesses cost one XOR with a constant each.
 template <int L>

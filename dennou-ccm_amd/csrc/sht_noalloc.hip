@@ -57,7 +57,7 @@ int sht_spec_to_grid_dev_noalloc(sht_plan *h, const double *spec, double *grid, 
   Plan &p = h->p;
   if (nf < 1 || nf > p.kmax)
     return fail(SHT_ERR_INVALID, "sht_spec_to_grid_dev_noalloc: nfield must be in [1, kmax]");
-  // the intermediate [P2][ceil(nf/G)][N+1][2][2G] in FP64, FP32 in the mixed forms
+  // the intermediate [ceil(nf/G)][P2][N+1][2][2G] in FP64, FP32 in the mixed forms:
   // the largest layout any shape of the call can use (the fused inverse
   // always takes the big FFT blocks)
   const FourGeom g = four_geom_g(p, fft_group(p.im), nf);

@@ -526,7 +526,8 @@ def restart_read(path, im: int, jm: int, km: int, nq: int = 1):
 
 class Batch:
     """Ensemble batch (sht_batch_*): members of uneven truncation and level
-    count, transformed by one graph launch.  members: list of
+    count, transformed by one launch per stage of all smaller grids, beside the
+    larger ones' own as branches of a graph.  members: list of
     (nmax, im, jm, nfield)."""
 
     def __init__(self, members, precision: int = PREC_FP64):

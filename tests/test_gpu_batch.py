@@ -1,5 +1,5 @@
 """Ensemble batches (sht_batch_*): members of uneven truncation and level count
-in one graph launch.  Each member's result must be bitwise the same as the same
+in shared launches and graph branches.  Each member's result must be bitwise the same as the same
 member transformed alone, and match the FP64 oracle (1e-12, or the mixed
 form's tolerance); graph replays must equal the eager run every time."""
 import numpy as np
